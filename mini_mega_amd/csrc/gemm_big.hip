@@ -18,7 +18,8 @@
 //     (through perm[] for L1, slot order for L2), converts them once to bf16
 //     with the row's UE8M0 scale folded in (exact), and stores them in a
 //     double-buffered LDS tile: [token tile][k-group q][lane][8 bf16], so that
-//     a wave's operand read for one MFMA group is 1 KiB contiguous;
+//     a wave's operand read for one MFMA group is 1 KiB contiguous (lanes
+//     permuted within it, see x_swizzle);
 //   * each wave streams its weight tiles (L1: gate and up rows of its hidden
 //     columns; L2: its output channels) from HBM through a 2- to 6-stage
 //     register pipeline and converts them exactly to bf16;
@@ -36,6 +37,7 @@
 // launch whose L2 units wait on per-item ready counters (reference:
 // src/compute_big.cuh:1948-1997).
 #include <type_traits>
+#include <utility>
 
 #include "mm_kernels.h"
 
@@ -47,7 +49,9 @@
 
 namespace mm {
 
-constexpr int kXTileBytes = 16 * kTileK * 2;   // one bf16 token tile: 16 rows x 128 k
+constexpr int kXOddPad = 16;   // LDS shift of the odd 16-byte columns (x_swizzle)
+constexpr int kXTileBytes = 16 * kTileK * 2 + kXOddPad;   // one bf16 token tile: 16 rows x 128 k
+constexpr int kXTile8Bytes = kTileBytes + kXOddPad;       // the same in fp8
 constexpr int kBlockTiles = 16;                 // weight tiles = 256 rows per workgroup
 constexpr int kBigRows = kBigMaxTiles * 16;     // token rows per work item (max)
 static_assert(kBlockTiles * 16 == kL2BlockN && kBlockTiles * 8 == kL1BlockH, "block shape");
@@ -72,14 +76,31 @@ struct alignas(16) BigSmem {
     uint8_t sfw[kBigMaxKT][kBlockTiles];        // the block's weight-tile scales [k-step][tile]
 };
 
-// Loader for NT active token tiles: chunk i = (tid + T*u) mod (NT*128), T
-// the workgroup's threads, is row r = 16*(i/128) + i%16 of the item, fp8
-// bytes [16*cc, 16*cc+16) of the k-step with cc = (i/16)%8: k-group g = cc/2,
-// MFMA groups q = 2*(cc%2) and q+1.  Rows vary fastest, so the 16 lanes of an
-// LDS write phase fill 16 consecutive 16-byte slots (no bank conflicts).
-// When NT*128 is not a multiple of T some threads redo another thread's
-// chunk (same bytes to the same LDS slot), which keeps every thread's work
-// uniform.  XS register stages: with two, the rows of k-step kt+2 are in
+// Row r (0..15) of a token tile sits in 16-byte slot r ^ x_swizzle(g) of the
+// 256 bytes of its k-group g (0..3), and the pieces of the odd 16-byte columns
+// start 16 bytes further (kXOddPad).  The loader's 8 consecutive lanes hold the
+// 8 columns cc = 2g + odd of one row, which the plain layout would put 256
+// bytes apart, in the same LDS banks; here they write 8 different slots (the
+// swizzles are even, the pad moves the odd columns to the slots between).
+// Bits 2 and 3 of every swizzle are equal: a ds_read_b128 serves a wave's lanes
+// in sets such as {0-3, 12-15, 20-27}, whose slots stay distinct only if no
+// k-group moves the slots {0-3, 12-15} into {4-11}.
+__device__ __forceinline__ constexpr int x_swizzle(int g) { return 2 * (g & 1) + 12 * (g >> 1); }
+
+// A lane's byte offset into the 1 KiB piece of its MFMA operand (row L%16,
+// k-group L/16), from lane16 = 16 * L.
+__device__ __forceinline__ uint32_t x_read_offset(uint32_t lane16) {
+    return lane16 ^ ((lane16 >> 3) & 0x60u) ^ ((lane16 >> 2) & 0x80u);
+}
+
+// Loader for NT active token tiles.  A thread's chunk u is 16 fp8 bytes, column
+// cc of one row of token tile tile(u): k-group g = cc/2, MFMA groups q =
+// 2*(cc%2) and q+1.  8 consecutive lanes read one row's 128 contiguous bytes,
+// a whole cache line.  (With the lanes of a quad on four rows, each load
+// looked up four times as many lines.  Measured on MI355X, T = 8192 fp8 MFMA
+// path with 256 rows per expert: the vL1D's accesses halved, L1 15% fewer
+// cycles.)
+// XS register stages: with two, the rows of k-step kt+2 are in
 // flight while kt+1 is written to LDS; with one (above 12 token tiles, where
 // registers go to accumulators, and a k-step's 4*NT MFMA groups alone cover
 // an L2 hit; measured even with two at T = 8192), kt+1 is loaded during kt.
@@ -91,6 +112,7 @@ struct XLoader {
     const uint8_t* base;
     int tid_;   // kOpaqueTid: the thread index, read once per unit through an empty asm
     uint32_t off[U];
+    uint32_t slot0, sfx0;   // the thread's chunk within a tile: LDS offset of its slot / its scales
     v4i reg[XS][U];
 
     __device__ __forceinline__ int tid() const {
@@ -105,39 +127,58 @@ struct XLoader {
     __device__ __forceinline__ int wave() const {
         return __builtin_amdgcn_readfirstlane(tid() >> 6);
     }
-    __device__ __forceinline__ int chunk(int u) const { return (tid() + kThreads * u) % (NT * 128); }
-    __device__ __forceinline__ static int row_of(int i) { return ((i >> 7) << 4) | (i & 15); }
-    __device__ __forceinline__ static int cc_of(int i) { return (i >> 4) & 7; }
-    __device__ __forceinline__ static int slot_of(int i) {
-        const int r = row_of(i), cc = cc_of(i);
-        return (r >> 4) * kXTileBytes + 2 * (cc & 1) * 1024 + ((r & 15) + 16 * (cc >> 1)) * 16;
+    // The token tile of chunk u, wave-uniform: two waves share a tile.  When
+    // NT is not a multiple of T / 128 some waves redo another's tile.
+    __device__ __forceinline__ int tile(int u) const {
+        return ((wave() >> 1) + kThreads / 128 * u) % NT;
     }
-
+    // Row within the tile and 16-byte column of the thread's chunks.  Columns
+    // vary fastest, and neighbouring groups of 8 lanes take rows 4 apart: the
+    // two swizzled rows of 16 lanes then cover all 16 slots.
+    __device__ __forceinline__ int row() const {
+        const int i = tid();
+        return ((i >> 4) & 3) | ((i >> 1) & 4) | ((i >> 3) & 8);
+    }
+    __device__ __forceinline__ int col() const { return tid() & 7; }
+    // row_off(r): byte offset of the item's row r (0..16*NT) from base
+    template <class RowOff>
+    __device__ __forceinline__ void init(RowOff row_off, int odd_bytes) {
+        const int r = row(), cc = col();
+#pragma unroll
+        for (int u = 0; u < U; ++u) off[u] = row_off(16 * tile(u) + r) + cc * 16;
+        slot0 = (cc & 1) * odd_bytes + ((r ^ x_swizzle(cc >> 1)) + 16 * (cc >> 1)) * 16;
+        sfx0 = r * kSfxPitch;
+    }
+    __device__ __forceinline__ void issue_one(int kt, int rs, int u) {
+        reg[rs][u] = load16_rows<kAux>(base, off[u], kt * kTileK);
+    }
     __device__ __forceinline__ void issue(int kt, int rs) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) reg[rs][u] = load16_rows<kAux>(base, off[u], kt * kTileK);
+        for (int u = 0; u < U; ++u) issue_one(kt, rs, u);
     }
-    // Writes chunk u of register stage rs, scaled by 2^(e - 127), to LDS stage xw.
-    __device__ __forceinline__ void commit_chunk(uint8_t* xw, int rs, int u, uint32_t e) {
-        uint8_t* t = xw + slot_of(chunk(u));
+    // The scale byte of chunk u's row at k-step kt.
+    __device__ __forceinline__ uint32_t scale(const BigSmem& sm, int u, int kt) const {
+        return (&sm.sfx[0][0])[sfx0 + (uint32_t)(tile(u) * 16 * kSfxPitch + kt)];
+    }
+    // Writes chunk u of register stage rs, scaled by 2^(e - 127), to the LDS
+    // stage at byte xw of sm.x.
+    __device__ __forceinline__ void commit_chunk(BigSmem& sm, uint32_t xw, int rs, int u,
+                                                 uint32_t e) {
+        uint8_t* t = &sm.x[0][0] + (slot0 + (xw + tile(u) * kXTileBytes));
         const float s = ue8m0_to_f32(e);
         *reinterpret_cast<v8bf*>(t) = fp8x8_to_bf16(reg[rs][u][0], reg[rs][u][1], s);
         *reinterpret_cast<v8bf*>(t + 1024) = fp8x8_to_bf16(reg[rs][u][2], reg[rs][u][3], s);
     }
-    __device__ __forceinline__ void commit(BigSmem& sm, int stage, int rs, int kt) {
+    __device__ __forceinline__ void commit(BigSmem& sm, int rs, int kt) {
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-            commit_chunk(&sm.x[stage][0], rs, u, sm.sfx[row_of(chunk(u))][kt]);
+        for (int u = 0; u < U; ++u) commit_chunk(sm, 0, rs, u, scale(sm, u, kt));
     }
     // fp8 MFMA path: the chunk's 16 raw bytes go to the fp8 token tile in the
-    // weight-tile layout ([half][lane][16 B], 2 KiB a tile), unconverted (the
-    // MFMA applies the row scale).
-    __device__ __forceinline__ static int slot_of_f8(int i) {
-        const int r = row_of(i), cc = cc_of(i);
-        return (r >> 4) * kTileBytes + (cc & 1) * 1024 + ((r & 15) + 16 * (cc >> 1)) * 16;
-    }
-    __device__ __forceinline__ void commit_chunk_f8(uint8_t* xw, int rs, int u) {
-        *reinterpret_cast<v4i*>(xw + slot_of_f8(chunk(u))) = reg[rs][u];
+    // weight-tile layout ([half][lane][16 B], swizzled), unconverted (the MFMA
+    // applies the row scale).
+    __device__ __forceinline__ void commit_chunk_f8(BigSmem& sm, uint32_t xw, int rs, int u) {
+        *reinterpret_cast<v4i*>(&sm.x[0][0] + (slot0 + (xw + tile(u) * kXTile8Bytes))) =
+            reg[rs][u];
     }
 };
 
@@ -146,14 +187,17 @@ struct WStage {
     v4i a[WT][2];   // the wave's weight tiles, two 16-byte halves each
 };
 
+// Half i & 1 of weight tile i / 2.
+template <int WT>
+__device__ __forceinline__ void w_load_half(WStage<WT>& w, const WTiles<WT>& wt, int kt, int i) {
+    w.a[i >> 1][i & 1] = load16_row_stream(wt.row[i >> 1], wt.KT * kTileBytes,
+                                           (int)wt.lane16 + 1024 * (i & 1), kt * kTileBytes);
+}
+
 template <int WT>
 __device__ __forceinline__ void w_load(WStage<WT>& w, const WTiles<WT>& wt, int kt) {
 #pragma unroll
-    for (int t = 0; t < WT; ++t) {
-        const int o = (int)wt.lane16, so = kt * kTileBytes;
-        w.a[t][0] = load16_row_stream(wt.row[t], wt.KT * kTileBytes, o, so);
-        w.a[t][1] = load16_row_stream(wt.row[t], wt.KT * kTileBytes, o + 1024, so);
-    }
+    for (int i = 0; i < 2 * WT; ++i) w_load_half<WT>(w, wt, kt, i);
 }
 
 // Weight tile t's operand of k-group q (8 bf16 per lane) with scale s folded in.
@@ -187,10 +231,10 @@ constexpr int big_stages() {
     return (W == 8 ? NT > 12 : NT > 8) ? 2 : (W == 8 && NT <= 8 && L2 ? 6 : 4);
 }
 
-// Activation operand reads in flight ahead of their MFMAs: 3, or 2 for W = 8
-// above NT = 12 (registers).
-template <int W, int NT>
-constexpr int big_read_ahead() { return (W == 8 && NT > 12) ? 2 : 3; }
+// Activation operand reads in flight ahead of their MFMAs (a ring of 4
+// operands; 4 divides the 4*NT chunks of a step, so that the ring's slots
+// line up from step to step).
+constexpr int kReadAhead = 3;
 
 // Bodies of at most this many token tiles issue their first weight stages
 // before the unit's scale staging, whose load round trip then overlaps the
@@ -214,29 +258,72 @@ struct NextW {
     bool has;
 };
 
+// f(0), f(1), .. f(N - 1), the index a compile-time constant in each call:
+// the k-steps' chunks differ in which loads, conversions and commits they
+// hold, and as a loop over run-time conditions the larger bodies passed the
+// compiler's limit for unrolling (the stages then went to scratch memory).
+template <class F, int... i>
+__device__ __forceinline__ void static_for_(F&& f, std::integer_sequence<int, i...>) {
+    (f(std::integral_constant<int, i>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+    static_for_(f, std::make_integer_sequence<int, N>{});
+}
+
+// The state that a k-step hands to the next one: the converted k-group-0
+// weight operand, the ring of activation operands (the first D chunks' are
+// already read), and the weight-tile scale bytes.
+template <int WT>
+struct StepCarry {
+    v8bf a0[WT];
+    v8bf b[4];
+    uint32_t sc;
+    uint32_t rd0;   // the lane's operand offset (x_read_offset)
+};
+
 // One k-step, software-pipelined by hand.  The step's 4*NT chunks (k-group
 // q, token tile j) each hold: the LDS read of the activation operand D
-// chunks ahead, a share of the conversions of the next k-group's weight
-// operands (in the last group: the next k-step's first), a share of the
-// activation commit of k-step kt+1 (last group only), and the chunk's kWT
-// MFMAs.  A scheduling fence closes every chunk, so the compiler keeps this
-// order: operand reads stay ahead of their use, and conversions overlap the
-// MFMAs instead of stalling them.  Before the chunks: the prefetches of
-// weights (kt+S-1) and activations (kt+XS), with indices clamped to the last
-// step (a redundant in-bounds reload keeps the loop free of branches, so the
-// compiler's wait counts stay partial).  After: the barrier that publishes
-// the committed activations.  a0 carries the converted k-group-0 operand from
-// one step to the next.
+// chunks ahead (across the step's end), a share of the conversions of the
+// next k-group's weight operands (in the last group: the next k-step's
+// first), now and then one of the step's vector loads (the vector-memory path
+// takes 16 cycles for each, from 8 waves at once), a share of the activation
+// commit of k-step kt+1 in the last chunks before the barrier, and the chunk's
+// kWT MFMAs.  A scheduling fence closes every chunk, so the
+// compiler keeps this order: operand reads stay ahead of their use, and the
+// conversions and loads overlap the MFMAs instead of stalling them.  The
+// loads are the weights of k-step kt+S-1 and the activations of kt+XS, with
+// indices clamped to the last step (a redundant in-bounds reload keeps the
+// loop free of branches, so the compiler's wait counts stay partial).  The
+// barrier that publishes the committed activations (and frees this step's
+// buffer: every wave's reads are done by then) stands before chunk kBar, D
+// chunks before the end, so that the next step's first operand reads run
+// under the last chunks' MFMAs.
+// What bounds it: at 16 token tiles the matrix cores are busy 67% of the
+// cycles, and power holds the clock at 1.9 GHz (MFMAs alone, on the same kind
+// of data, run at 2.15 GHz).  So instructions and LDS accesses saved count
+// even where they overlap, and deeper prefetch does not: 7 operand reads
+// ahead, 3 weight stages or 2 activation stages above 12 tiles were all even.
+// Measured on MI355X (L1 / L2 us, 256 experts, H = 6144, I = 2048, equal rows
+// per expert) against a step that issued all loads first and ended on the
+// barrier, with the rows gathered 64 bytes at a time: 16 rows 943 / 530 ->
+// 936 / 527, 64 rows 1099 / 584 -> 1040 / 572, 256 rows 2668 / 1416 -> 2565 /
+// 1367, 288 rows (two items of 9 tiles) 3271 / 1788 -> 3130 / 1710.
 template <int W, int NT, int S, int s, class XL, class NX = NoNext>
 __device__ __forceinline__ void big_step(v4f (&acc)[Geo<W>::kWT][NT], BigSmem& sm,
                                          XL& xl, WStage<Geo<W>::kWT> (&w)[S],
-                                         const WTiles<Geo<W>::kWT>& wt, v8bf (&a0)[Geo<W>::kWT],
+                                         const WTiles<Geo<W>::kWT>& wt,
+                                         StepCarry<Geo<W>::kWT>& cy,
                                          int kt, int KT, const NX& nx = NX{}) {
     constexpr int kWT = Geo<W>::kWT;
     constexpr int XS = XL::XS, U = XL::U;
-    constexpr int G = 4 * NT, D = big_read_ahead<W, NT>() < G ? big_read_ahead<W, NT>() : G;
+    constexpr int G = 4 * NT, D = kReadAhead;
+    constexpr int kBar = G - D;
+    constexpr int kLoads = 2 * kWT + U;               // vector loads of the step
+    constexpr int kSpread = NX::kOn ? 1 : NT <= 2 ? NT : 2 * NT;   // .. issued over these chunks
+    constexpr int kCommit = kBar - NT > 0 ? kBar - NT : 0, kCommitN = kBar - kCommit;
     constexpr int rs = XS == 2 ? ((s + 1) & 1) : 0;   // register stage holding k-step kt+1
-    const int lane = xl.tid() & 63, wave = xl.wave();
+    const int wave = xl.wave();
     // weights first: vector loads complete in issue order, so the wait for
     // the next step's weights (end of this step) must not also wait for this
     // step's gathered activation rows, which can miss to HBM (measured:
@@ -244,92 +331,103 @@ __device__ __forceinline__ void big_step(v4f (&acc)[Geo<W>::kWT][NT], BigSmem& s
     // when walking (L2 units only): the activation rows first, so that the
     // commit's wait does not also wait for the weights issued ahead of them
     // (measured on MI355X with the walk at T = 2048: L2 610-611 vs 615-618 us)
-    if constexpr (NX::kOn) xl.issue(min(kt + XS, KT - 1), XS == 2 ? (s & 1) : 0);
+    int kw = min(kt + S - 1, KT - 1);
+    WTiles<kWT> ws = wt;
     if constexpr (NX::kOn) {
-        const int kw = kt + S - 1;
-        const bool cur = kw < KT, nxt = !cur && nx.has;
-        WTiles<kWT> ws = wt;
+        const bool cur = kt + S - 1 < KT, nxt = !cur && nx.has;
 #pragma unroll
         for (int t = 0; t < kWT; ++t) ws.row[t] = nxt ? nx.wt.row[t] : wt.row[t];
-        w_load<kWT>(w[(s + S - 1) % S], ws, cur ? kw : nxt ? kw - KT : KT - 1);
-    } else {
-        w_load<kWT>(w[(s + S - 1) % S], wt, min(kt + S - 1, KT - 1));
+        kw = cur ? kt + S - 1 : nxt ? kt + S - 1 - KT : KT - 1;
     }
-    if constexpr (!NX::kOn) xl.issue(min(kt + XS, KT - 1), XS == 2 ? (s & 1) : 0);
-    // scale bytes, read here and decoded where used (no wait before the MFMAs)
+    auto load = [&](int i) {
+        constexpr int xfirst = NX::kOn ? U : 0;   // the activations come first
+        if (NX::kOn ? i < U : i >= 2 * kWT)
+            xl.issue_one(min(kt + XS, KT - 1), XS == 2 ? (s & 1) : 0, NX::kOn ? i : i - 2 * kWT);
+        else
+            w_load_half<kWT>(w[(s + S - 1) % S], ws, kw, i - xfirst);
+    };
     const int kn = min(kt + 1, KT - 1);
-    const uint32_t sc = w_scales<kWT>(sm, kt, wave), sn = w_scales<kWT>(sm, kn, wave);
-    uint32_t xs[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-        xs[u] = sm.sfx[XL::row_of(xl.chunk(u))][kn];
+    const uint32_t sc = cy.sc;
     // LDS bases of this step's read and write buffers.  Opaque to the
     // optimiser: otherwise it hoists every operand address of the unrolled
     // group out of the loop into a register of its own (the buffer parity of
     // each step is known there) instead of using one base plus immediate
     // offsets.
-    uint32_t xro = (kt & 1) * (uint32_t)sizeof(sm.x[0]) + lane * 16;
-    uint32_t xwo = ((kt + 1) & 1) * (uint32_t)sizeof(sm.x[0]);
-    asm volatile("" : "+v"(xro), "+v"(xwo));
-    const uint8_t* xb = &sm.x[0][0] + xro;
-    uint8_t* xw = &sm.x[0][0] + xwo;
-    v8bf b[D + 1];
-#pragma unroll
-    for (int d = 0; d < D; ++d)
-        b[d] = *reinterpret_cast<const v8bf*>(xb + (d % NT) * kXTileBytes + (d / NT) * 1024);
-    __builtin_amdgcn_sched_barrier(0);
+    uint32_t xrs = (kt & 1) * (uint32_t)sizeof(sm.x[0]);
+    uint32_t xws = (uint32_t)sizeof(sm.x[0]) - xrs;
+    asm volatile("" : "+s"(xrs), "+s"(xws));
+    const uint32_t xro = cy.rd0 + xrs, xno = cy.rd0 + xws;   // this step's and the next one's
+    auto rd = [&](uint32_t base, int slot, int g) {   // chunk g's operand
+        const int q = g / NT;
+        cy.b[slot] = *reinterpret_cast<const v8bf*>(
+            &sm.x[0][0] + base + (g % NT) * kXTileBytes + q * 1024 + (q >> 1) * kXOddPad);
+    };
+    uint32_t sn = 0, xs[U];
     v8bf ac[kWT], an[kWT];
 #pragma unroll
-    for (int t = 0; t < kWT; ++t) ac[t] = a0[t];
+    for (int t = 0; t < kWT; ++t) ac[t] = cy.a0[t];
+    static_for<G>([&](auto gc) {
+        constexpr int g = gc, q = g / NT, j = g % NT;
+        if constexpr (g == kBar) __syncthreads();
+        if constexpr (g + D < G)
+            rd(xro, (g + D) & 3, g + D);
+        else
+            rd(xno, (g + D) & 3, g + D - G);
+        if constexpr (g == 0) {
+            sn = w_scales<kWT>(sm, kn, wave);
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-        const int q = g / NT, j = g % NT;
-        if (g + D < G) {
-            const int gn = g + D;
-            b[gn % (D + 1)] = *reinterpret_cast<const v8bf*>(xb + (gn % NT) * kXTileBytes +
-                                                             (gn / NT) * 1024);
+            for (int u = 0; u < U; ++u) xs[u] = xl.scale(sm, u, kn);
         }
-#pragma unroll
-        for (int t = 0; t < kWT; ++t)
-            if (j == (t * NT) / kWT)
+        static_for<kLoads>([&](auto i) {
+            if constexpr (g == (i * kSpread) / kLoads) load(i);
+        });
+        static_for<kWT>([&](auto tc) {
+            constexpr int t = tc;
+            if constexpr (j == (t * NT) / kWT)
                 an[t] = q < 3 ? w_group<kWT>(w[s], t, q + 1, scale_of(sc, t))
                               : w_group<kWT>(w[(s + 1) % S], t, 0, scale_of(sn, t));
-        if (q == 3) {
+        });
+        static_for<U>([&](auto uc) {
+            constexpr int u = uc;
+            if constexpr (g == kCommit + (u * kCommitN) / U)
+                xl.commit_chunk(sm, xws, rs, u, xs[u]);
+        });
+        // odd chunks in reverse: one operand stays the same from one MFMA to
+        // the next, also across the chunks
 #pragma unroll
-            for (int u = 0; u < U; ++u)
-                if (j == (u * NT) / U) xl.commit_chunk(xw, rs, u, xs[u]);
+        for (int i = 0; i < kWT; ++i) {
+            const int t = g & 1 ? kWT - 1 - i : i;
+            acc[t][j] = mfma_bf16(ac[t], cy.b[g & 3], acc[t][j]);
         }
-#pragma unroll
-        for (int t = 0; t < kWT; ++t) acc[t][j] = mfma_bf16(ac[t], b[g % (D + 1)], acc[t][j]);
-        if (j == NT - 1) {
+        if constexpr (j == NT - 1) {
 #pragma unroll
             for (int t = 0; t < kWT; ++t) ac[t] = an[t];
         }
         __builtin_amdgcn_sched_barrier(0);
-    }
+    });
 #pragma unroll
-    for (int t = 0; t < kWT; ++t) a0[t] = ac[t];
-    __syncthreads();
+    for (int t = 0; t < kWT; ++t) cy.a0[t] = ac[t];
+    cy.sc = sn;
 }
 
 template <int W, int NT, int S, int s, class XL, class NX>
 __device__ __forceinline__ void big_group(v4f (&acc)[Geo<W>::kWT][NT], BigSmem& sm,
                                           XL& xl, WStage<Geo<W>::kWT> (&w)[S],
-                                          const WTiles<Geo<W>::kWT>& wt, v8bf (&a0)[Geo<W>::kWT],
-                                          int kb, int KT, const NX& nx) {
-    big_step<W, NT, S, s>(acc, sm, xl, w, wt, a0, kb + s, KT, nx);
-    if constexpr (s + 1 < S) big_group<W, NT, S, s + 1>(acc, sm, xl, w, wt, a0, kb, KT, nx);
+                                          const WTiles<Geo<W>::kWT>& wt,
+                                          StepCarry<Geo<W>::kWT>& cy, int kb, int KT, const NX& nx) {
+    big_step<W, NT, S, s>(acc, sm, xl, w, wt, cy, kb + s, KT, nx);
+    if constexpr (s + 1 < S) big_group<W, NT, S, s + 1>(acc, sm, xl, w, wt, cy, kb, KT, nx);
 }
 
 // The KT % S remaining k-steps, one guarded step each.
 template <int W, int NT, int S, int r, class XL, class NX>
 __device__ __forceinline__ void big_tail(v4f (&acc)[Geo<W>::kWT][NT], BigSmem& sm,
                                          XL& xl, WStage<Geo<W>::kWT> (&w)[S],
-                                         const WTiles<Geo<W>::kWT>& wt, v8bf (&a0)[Geo<W>::kWT],
-                                         int KF, int KT, const NX& nx) {
+                                         const WTiles<Geo<W>::kWT>& wt,
+                                         StepCarry<Geo<W>::kWT>& cy, int KF, int KT, const NX& nx) {
     if (KF + r < KT) {
-        big_step<W, NT, S, r>(acc, sm, xl, w, wt, a0, KF + r, KT, nx);
-        if constexpr (r + 2 < S) big_tail<W, NT, S, r + 1>(acc, sm, xl, w, wt, a0, KF, KT, nx);
+        big_step<W, NT, S, r>(acc, sm, xl, w, wt, cy, KF + r, KT, nx);
+        if constexpr (r + 2 < S) big_tail<W, NT, S, r + 1>(acc, sm, xl, w, wt, cy, KF, KT, nx);
     }
 }
 
@@ -370,18 +468,22 @@ __device__ __forceinline__ void big_mainloop(v4f (&acc)[Geo<W>::kWT][NT], BigSme
     } else if constexpr (!kEarly) {
         w_prologue<kWT, S>(w, wt, KT);
     }
-    xl.commit(sm, 0, 0, 0);
+    xl.commit(sm, 0, 0);
     __syncthreads();
-    v8bf a0[kWT];
-    {
-        const uint32_t sc = w_scales<kWT>(sm, 0, xl.wave());
+    StepCarry<kWT> cy;
+    cy.sc = w_scales<kWT>(sm, 0, xl.wave());
+    cy.rd0 = x_read_offset(wt.lane16);
 #pragma unroll
-        for (int t = 0; t < kWT; ++t) a0[t] = w_group<kWT>(w[0], t, 0, scale_of(sc, t));
-    }
+    for (int g = 0; g < kReadAhead; ++g)
+        cy.b[g] = *reinterpret_cast<const v8bf*>(
+            &sm.x[0][0] + cy.rd0 + (g % NT) * kXTileBytes + (g / NT) * 1024 +
+            (g / NT >> 1) * kXOddPad);
+#pragma unroll
+    for (int t = 0; t < kWT; ++t) cy.a0[t] = w_group<kWT>(w[0], t, 0, scale_of(cy.sc, t));
     const int KF = KT - KT % S;
 #pragma unroll 1
-    for (int kb = 0; kb < KF; kb += S) big_group<W, NT, S, 0>(acc, sm, xl, w, wt, a0, kb, KT, nx);
-    big_tail<W, NT, S, 0>(acc, sm, xl, w, wt, a0, KF, KT, nx);
+    for (int kb = 0; kb < KF; kb += S) big_group<W, NT, S, 0>(acc, sm, xl, w, wt, cy, kb, KT, nx);
+    big_tail<W, NT, S, 0>(acc, sm, xl, w, wt, cy, KF, KT, nx);
 }
 
 // ---------------------------------------------------------- fp8 MFMA path --
@@ -444,18 +546,19 @@ __device__ __forceinline__ void big_step_f8(v4f (&acc)[Geo<W>::kWT][NT], BigSmem
     w_load8<kWT>(w[(s + S - 1) % S], wt, min(kt + S - 1, KT - 1));   // s: step in the group
     xl.issue(min(kt + XS, KT - 1), XS == 2 ? (s & 1) : 0);
     const uint32_t sc = w_scales<kWT>(sm, kt, wave);
-    uint32_t xro = (kt & 1) * (uint32_t)sizeof(sm.x[0]) + lane * 16;
-    uint32_t xwo = ((kt + 1) & 1) * (uint32_t)sizeof(sm.x[0]);
-    uint32_t sfo = (lane & 15) * kSfxPitch + kt;
-    asm volatile("" : "+v"(xro), "+v"(xwo), "+v"(sfo));
+    uint32_t xro = x_read_offset(wt.lane16), sfo = (lane & 15) * kSfxPitch;
+    uint32_t xrs = (kt & 1) * (uint32_t)sizeof(sm.x[0]);
+    uint32_t xws = (uint32_t)sizeof(sm.x[0]) - xrs;
+    asm volatile("" : "+s"(xrs), "+s"(xws));
+    xro += xrs;
+    sfo += kt;
     const uint8_t* xb = &sm.x[0][0] + xro;
-    uint8_t* xw = &sm.x[0][0] + xwo;
     const uint8_t* sf = &sm.sfx[0][0] + sfo;
     v8i b[D + 1];
     uint32_t bs[D + 1];
     auto rd = [&](int d, int j) {
-        const v4i lo = *reinterpret_cast<const v4i*>(xb + j * kTileBytes);
-        const v4i hi = *reinterpret_cast<const v4i*>(xb + j * kTileBytes + 1024);
+        const v4i lo = *reinterpret_cast<const v4i*>(xb + j * kXTile8Bytes);
+        const v4i hi = *reinterpret_cast<const v4i*>(xb + j * kXTile8Bytes + 1024 + kXOddPad);
         b[d] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
         bs[d] = sf[j * 16 * kSfxPitch];
     };
@@ -467,7 +570,7 @@ __device__ __forceinline__ void big_step_f8(v4f (&acc)[Geo<W>::kWT][NT], BigSmem
         if (j + D < NT) rd((j + D) % (D + 1), j + D);
 #pragma unroll
         for (int u = 0; u < U; ++u)
-            if (j == (u * NT) / U) xl.commit_chunk_f8(xw, rs, u);
+            if (j == (u * NT) / U) xl.commit_chunk_f8(sm, xws, rs, u);
 #pragma unroll
         for (int t = 0; t < kWT; ++t)
             acc[t][j] = mfma_f8(w[s % S].a[t], b[j % (D + 1)], (sc >> (8 * t)) & 0xffu,
@@ -516,7 +619,7 @@ __device__ __forceinline__ void big_mainloop_f8(v4f (&acc)[Geo<W>::kWT][NT], Big
         for (int st = 0; st < S - 1; ++st) w_load8<kWT>(w[st], wt, min(st, KT - 1));
     }
 #pragma unroll
-    for (int u = 0; u < U; ++u) xl.commit_chunk_f8(&sm.x[0][0], 0, u);
+    for (int u = 0; u < U; ++u) xl.commit_chunk_f8(sm, 0, 0, u);
     __syncthreads();
     const int KF = KT - KT % GS;
 #pragma unroll 1
@@ -688,17 +791,6 @@ __device__ __forceinline__ void big_load_scales(BigSmem& sm, int KT, int nrows, 
         default: BODY(16); break; \
     }
 
-// Sets the loader's row offsets: row r of the item (r >= rows: row 0,
-// whose bytes are loaded but whose results are never stored).
-template <class XL, class RowOff>
-__device__ __forceinline__ void big_loader_init(XL& xl, RowOff row_off) {
-#pragma unroll
-    for (int u = 0; u < XL::U; ++u) {
-        const int i = xl.chunk(u);
-        xl.off[u] = row_off(XL::row_of(i)) + XL::cc_of(i) * 16;
-    }
-}
-
 // ---------------------------------------------------------------------- L1 --
 // Block tile bt = kWT*wave + t of an L1 block: the wave's hidden columns are
 // hw0 = bx*128 + wave*(128/W) .. +128/W; tiles t < kWT/2 are the gate rows of
@@ -755,7 +847,7 @@ __device__ __forceinline__ void l1_big_body(const GemmParams& p, const BigItem& 
     // one stage above 10 tiles)
     XLoader<W, NT, 0, false, (kF8 || NT <= 12 ? 2 : 1)> xl;
     xl.base = p.x;
-    big_loader_init(xl, [&](int r) { return sm.tok[r] * (uint32_t)H; });
+    xl.init([&](int r) { return sm.tok[r] * (uint32_t)H; }, (kF8 ? 1024 : 2048) + kXOddPad);
     v4f acc[kWT][NT];
     if constexpr (kF8)
         big_mainloop_f8<W, NT, S, kEarly>(acc, sm, xl, wt, KT, w);
@@ -952,9 +1044,9 @@ __device__ __forceinline__ void l2_big_body(const GemmParams& p, const BigItem& 
     stage_scales();
     XLoader<W, NT, kFused ? kBufferSc1 : 0, false, (kF8 || NT <= 12 ? 2 : 1)> xl;
     xl.base = p.x;
-    big_loader_init(xl, [&](int r) {
-        return (uint32_t)(it.m0 + (r < it.rows ? r : 0)) * (uint32_t)I;
-    });
+    xl.init([&](int r) {
+        return (uint32_t)(it.m0 + (r < it.rows ? r : 0)) * (uint32_t)I;   // row 0 past the item's end
+    }, (kF8 ? 1024 : 2048) + kXOddPad);
     if constexpr (kF8)
         big_mainloop_f8<W, NT, S, kEarly>(acc, sm, xl, wt, KT, w);
     else
@@ -1101,9 +1193,9 @@ __device__ __forceinline__ void l2_walk_body(const GemmParams& p, const BigItem&
     XLoader<W, NT, 0, true> xl;
     xl.base = p.x;
     xl.tid_ = tid;
-    big_loader_init(xl, [&](int r) {
-        return (uint32_t)(it.m0 + (r < it.rows ? r : 0)) * (uint32_t)I;
-    });
+    xl.init([&](int r) {
+        return (uint32_t)(it.m0 + (r < it.rows ? r : 0)) * (uint32_t)I;   // row 0 past the item's end
+    }, 2048 + kXOddPad);
     v4f acc[kWT][NT];
     big_mainloop<W, NT, S, false>(acc, sm, xl, wt, KT, ring, nx, pref);
     l2_store_tile<W, NT>(p, it, sm, acc, it.bx * kL2BlockN, lane, wave);
