@@ -22,8 +22,10 @@ template <bool kStreamRows>
 __global__ void __launch_bounds__(1024)
 combine_kernel(const uint16_t* __restrict__ l2, const int* __restrict__ pair_pos,
                const float* __restrict__ w, int topk, int H, float* __restrict__ y,
-               uint16_t* __restrict__ y_bf16) {
+               uint16_t* __restrict__ y_bf16, int* __restrict__ l2_queue) {
 #pragma clang fp contract(off)
+    // the L2 GEMM has ended: its tail queue is zeroed for the next launch
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < kQueueInts) l2_queue[threadIdx.x] = 0;
     constexpr int kG = 8;
     const int t = blockIdx.x;
     const int c0 = (blockIdx.y * blockDim.x + threadIdx.x) * 8;
@@ -78,8 +80,8 @@ combine_kernel(const uint16_t* __restrict__ l2, const int* __restrict__ pair_pos
 }
 
 template __global__ void combine_kernel<false>(const uint16_t*, const int*, const float*, int, int,
-                                               float*, uint16_t*);
+                                               float*, uint16_t*, int*);
 template __global__ void combine_kernel<true>(const uint16_t*, const int*, const float*, int, int,
-                                              float*, uint16_t*);
+                                              float*, uint16_t*, int*);
 
 }  // namespace mm

@@ -642,17 +642,21 @@ struct BigItem {
 // equal modelled cost, and the XCDs take workgroups round-robin: workgroup L
 // is the k-th of XCD x = L%8, k = L/8 (measured on MI355X with the XCC_ID
 // register: every workgroup ran on XCD L%8).
-// Static bulk, dynamic tail.  While k < (range of x) - kQueueTail, workgroup
+// Static bulk, dynamic tail.  While k < (range of x) - tail_units, workgroup
 // L runs unit cuts[x] + k, with no atomic on its way to its first load.  The
-// last kQueueTail units of each range go out by ticket from that XCD's
+// last tail_units of each range go out by ticket from that XCD's
 // counter, to its workgroups k < range; the next kStealers workgroups of the
 // XCD take tickets from the other XCDs' tails, so that an XCD that runs
 // ahead of its modelled cost finishes the others' last units instead of
-// idling.  Every later workgroup exits at once: the grid (nb * max_items +
-// 8) is sized for the largest item count, and a surplus workgroup that paid
+// idling.  Every later workgroup exits at once: the grid is sized for the
+// largest item count, and a surplus workgroup that paid
 // atomics while holding a CU's LDS delayed the real tail (L2 650 -> 900 us
-// at T = 2048).  The last ticket taker of a launch zeroes the counters for
-// the next one.  Measured on MI355X (time-stamped workgroups): without the
+// at T = 2048).  The counters are zeroed by the next launch on the stream (the
+// other GEMM's, the combine's), or by the last ticket taker of a GEMM that is
+// launched alone: counting the takers costs each one more atomic, all on one
+// word, before its unit starts (measured on MI355X, 64 experts, H = 2048, I =
+// 768, T = 777: L2 52.4 us with it, 38.7 without).
+// Measured on MI355X (time-stamped workgroups): without the
 // queue the XCDs' last L1 units ended up to 55 us apart at T = 512, 175 us
 // at T = 8192 and 120 us with Zipf(1.1) skew; with it 22, 55 and 91 us.  A
 // stolen unit runs without the victim XCD's L2 contents, so the kernel span
@@ -668,29 +672,56 @@ struct BigItem {
 // Zipf(1.1) T = 2048 L1 1193-1195 vs 1223-1231 us, T = 512 / 2048 / 8192
 // even (measured on MI355X).  L2's tickets gained nothing from the order
 // and go out in unit order.
+// A range of at most two units per CU has no tail queue: its tickets cost more
+// than they balance (measured on MI355X, 64 experts, H = 2048, I = 768, T =
+// 777: L2, 64 units of 6 k-steps per XCD, 38.3 us with tickets, 34.1 without).
+__device__ __forceinline__ int tail_units(int range) {
+    return range > 2 * kQueueTail ? kQueueTail : 0;
+}
+
 __device__ __forceinline__ int claim_tail_unit(const GemmParams& p, int x, bool own, int grid) {
     int u = -1;
-    for (int d = own ? 0 : 1; d < 8 && u < 0; ++d) {
-        const int xx = (x + d) & 7;
-        const int lo = p.xcd_cuts[xx], hi = p.xcd_cuts[xx + 1];
-        const int tail = min(hi - lo, kQueueTail);
-        if (tail <= 0) continue;
+    auto take = [&](int xx) {
+        const int lo = p.xcd_cuts[xx], hi = p.xcd_cuts[xx + 1], tail = tail_units(hi - lo);
         const int t = atomicAdd(&p.queue[xx], 1);
         if (t < tail) u = hi - tail + (p.tail_ord ? p.tail_ord[kQueueTail * xx + t] : t);
-    }
-    // ticket takers of this launch: per XCD, its workgroups from the tail
-    // through its stealers (as many as the grid holds)
-    int takers = 0;
-    for (int xx = 0; xx < 8; ++xx) {
-        const int range = p.xcd_cuts[xx + 1] - p.xcd_cuts[xx];
-        const int wgs = (grid - xx + 7) >> 3;
-        takers += min(wgs, range + kStealers) - (range - min(range, kQueueTail));
-    }
-    if (atomicAdd(&p.queue[8], 1) == takers - 1) {
+    };
+    if (own) take(x);
+    if (u < 0) {
+        // the other XCDs' counters in one round trip; then only those with
+        // tickets left are asked
+        int c[8];
 #pragma unroll
-        for (int i = 0; i < kQueueInts; ++i) p.queue[i] = 0;
+        for (int xx = 0; xx < 8; ++xx)
+            c[xx] = __hip_atomic_load(&p.queue[xx], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        uint32_t left = 0;
+#pragma unroll
+        for (int xx = 0; xx < 8; ++xx)
+            if (xx != x && c[xx] < tail_units(p.xcd_cuts[xx + 1] - p.xcd_cuts[xx]))
+                left |= 1u << xx;
+        for (int d = 1; d < 8 && u < 0; ++d)
+            if (left >> ((x + d) & 7) & 1) take((x + d) & 7);
+    }
+    if (p.self_reset) {
+        // ticket takers of this launch: per XCD, its workgroups from the tail
+        // through its stealers (as many as the grid holds)
+        int takers = 0;
+        for (int xx = 0; xx < 8; ++xx) {
+            const int range = p.xcd_cuts[xx + 1] - p.xcd_cuts[xx];
+            const int wgs = (grid - xx + 7) >> 3;
+            takers += min(wgs, range + kStealers) - (range - tail_units(range));
+        }
+        if (atomicAdd(&p.queue[8], 1) == takers - 1) {
+#pragma unroll
+            for (int i = 0; i < kQueueInts; ++i) p.queue[i] = 0;
+        }
     }
     return u;
+}
+
+// Zeroes the other GEMM's tail queue (that launch has ended).
+__device__ __forceinline__ void reset_other_queue(const GemmParams& p) {
+    if (blockIdx.x == 0 && threadIdx.x < kQueueInts) p.other_queue[threadIdx.x] = 0;
 }
 
 // Workgroup L of a grid of `grid` (the big GEMM's own share of the launch).
@@ -705,7 +736,7 @@ __device__ __forceinline__ bool big_unit(const GemmParams& p, int nb, BigItem& i
     } else if (k >= range + kStealers) {
         return false;
     }
-    if (kTailQueue && k >= range - min(range, kQueueTail)) {
+    if (kTailQueue && k >= range - tail_units(range)) {
         if (threadIdx.x == 0) *s_unit = claim_tail_unit(p, x, k < range, grid);
         __syncthreads();
         u = *s_unit;
@@ -963,12 +994,14 @@ __device__ __forceinline__ void l1_big(const GemmParams& p, BigSmem& sm, int* s_
 __global__ void __launch_bounds__(512) l1_big_kernel(GemmParams p) {
     __shared__ BigSmem sm;
     __shared__ int s_unit;
+    reset_other_queue(p);
     l1_big<8, false>(p, sm, &s_unit, blockIdx.x, gridDim.x);
 }
 
 __global__ void __launch_bounds__(512) l1_big_f8_kernel(GemmParams p) {
     __shared__ BigSmem sm;
     __shared__ int s_unit;
+    reset_other_queue(p);
     l1_big<8, false, true>(p, sm, &s_unit, blockIdx.x, gridDim.x);
 }
 
@@ -1106,16 +1139,10 @@ __device__ __forceinline__ void l2_big(const GemmParams& p, BigSmem& sm, int* s_
 #undef MM_L2_BODY
 }
 
-__global__ void __launch_bounds__(512) l2_big_kernel(GemmParams p) {
-    __shared__ BigSmem sm;
-    __shared__ int s_unit;
-    if (walk_taken(p)) return;   // the walk (launched just before) ran the units
-    l2_big<8, false>(p, sm, &s_unit, blockIdx.x, gridDim.x);
-}
-
 __global__ void __launch_bounds__(512) l2_big_f8_kernel(GemmParams p) {
     __shared__ BigSmem sm;
     __shared__ int s_unit;
+    reset_other_queue(p);
     l2_big<8, false, true>(p, sm, &s_unit, blockIdx.x, gridDim.x);
 }
 
@@ -1240,10 +1267,17 @@ __device__ __forceinline__ void l2_walk(const GemmParams& p, BigSmem& sm, int L,
     }
 }
 
-__global__ void __launch_bounds__(512) l2_walk_kernel(GemmParams p) {
+// The launch's units as the walk (the first p.walk workgroups) or one unit
+// per workgroup.
+__global__ void __launch_bounds__(512) l2_big_kernel(GemmParams p) {
     __shared__ BigSmem sm;
-    if (!walk_taken(p)) return;   // l2_big_kernel, launched next, runs the units
-    l2_walk<8>(p, sm, blockIdx.x, gridDim.x);
+    __shared__ int s_unit;
+    reset_other_queue(p);
+    if (walk_taken(p)) {
+        if ((int)blockIdx.x < p.walk) l2_walk<8>(p, sm, blockIdx.x, p.walk);
+    } else {
+        l2_big<8, false>(p, sm, &s_unit, blockIdx.x, gridDim.x);
+    }
 }
 
 // L1 and L2 in one launch: workgroups [0, g1) run L1 units, the rest L2

@@ -7,6 +7,7 @@
 // synchronises: every launch entry point only validates its arguments and
 // enqueues kernels on `stream`, so the layer is capture-safe.  The workspace
 // is caller-owned, or (mm_launch_full_noalloc) the file-scope `scratch`.
+#include <algorithm>
 #include <cstddef>
 #include <cstdio>
 #include <cstdlib>
@@ -196,23 +197,48 @@ int cu_count() {
     return cached[dev];
 }
 
+// Workgroups of a big GEMM's launch (nb blocks per item).  The general grid,
+// nb * max_items + 8, covers whatever routing the workspace holds.  When this
+// call's own prologue made the routing (`routed`), its tokens bound the items
+// (at most min(E, P) experts, P / m_tile items more) and so each XCD's range:
+// the ranges are cut at equal cost, a unit costs 9 to cmax, so a range holds
+// at most 1/8 of the units' largest cost, and one unit at either end, over 9.
+// A launch of few tokens on a large workspace then dispatches no thousands of
+// workgroups that find no unit (measured on MI355X at T = 1 in a workspace
+// for 512 tokens: L1 42.1 -> 40.6 us, L2 21.0 -> 20.4).
+int big_grid(const MegaLaunchArgs& a, const Bound& b, int nb, bool routed) {
+    const int64_t full = (int64_t)nb * b.L.max_items + 8;
+    if (!routed) return (int)full;
+    const int64_t P = (int64_t)a.tokens * a.topk;
+    const int64_t items = std::min<int64_t>(a.num_experts, P) + P / b.m_tile;
+    const int64_t tiles = (std::min<int64_t>(P, b.m_tile) + 15) / 16;
+    const int64_t cmax = std::max<int64_t>(9, 2 + std::min<int64_t>(tiles, mm::kBigMaxTiles));
+    const int64_t range = (nb * items * cmax / 8 + cmax) / 9 + 1;
+    return (int)std::min(full, 8 * (range + mm::kStealers));
+}
+
 // Decode-shaped kernels (MT = 1, 2) for m_tile <= 32; above, the LDS-staged
-// kernels on a 1-D grid of nb * max_items + 8 workgroups (the kernel maps
-// workgroups to (item, block) units XCD by XCD and drops the surplus).
+// kernels on a 1-D grid (the kernel maps workgroups to (item, block) units XCD
+// by XCD and drops the surplus).
 void launch_gemm(const GemmKernel (&small)[2], GemmKernel big, int m_tile, int nb,
-                 int max_items, hipStream_t s, const mm::GemmParams& p) {
+                 int max_items, int grid, hipStream_t s, const mm::GemmParams& p) {
     if (m_tile <= 32) {
         hipLaunchKernelGGL(small[m_tile <= 16 ? 0 : 1], dim3(nb, max_items),
                            dim3(mm::kGemmThreads), 0, s, p);
     } else {
-        hipLaunchKernelGGL(big, dim3(nb * max_items + 8), dim3(mm::kBigThreads), 0, s, p);
+        hipLaunchKernelGGL(big, dim3(grid), dim3(mm::kBigThreads), 0, s, p);
     }
 }
 
 const GemmKernel kL1Small[2] = {mm::l1_kernel<1>, mm::l1_kernel<2>};
 const GemmKernel kL2Small[2] = {mm::l2_kernel<1>, mm::l2_kernel<2>};
 
-int do_l1(const MegaLaunchArgs& a, hipStream_t s) {
+// How a GEMM is launched: alone (an entry point of its own), or in
+// launch_compute, behind this call's own prologue (kRouted) or reusing the
+// previous one's routing.
+enum class Stage { kAlone, kReused, kRouted };
+
+int do_l1(const MegaLaunchArgs& a, Stage stage, hipStream_t s) {
     Bound b;
     int st = bind(a, b, true);
     if (st != kOk) return st;
@@ -226,14 +252,16 @@ int do_l1(const MegaLaunchArgs& a, hipStream_t s) {
     p.out_sf = b.ws + b.L.ffn_sf;
     p.xcd_cuts = p.status + mm::kCutsL1;
     p.queue = at<int>(b, b.L.status) + mm::kQueueL1;
+    p.other_queue = at<int>(b, b.L.status) + mm::kQueueL2;
+    p.self_reset = stage == Stage::kAlone;
     p.tail_ord = reinterpret_cast<const uint8_t*>(p.status + mm::kTailOrdL1);
     const int nb = a.intermediate / mm::kL1BlockH;
     launch_gemm(kL1Small, a.mfma_fp8 ? mm::l1_big_f8_kernel : mm::l1_big_kernel, b.m_tile, nb,
-                b.L.max_items, s, p);
+                b.L.max_items, big_grid(a, b, nb, stage == Stage::kRouted), s, p);
     return launched(kOk);
 }
 
-int do_l2(const MegaLaunchArgs& a, hipStream_t s) {
+int do_l2(const MegaLaunchArgs& a, Stage stage, hipStream_t s) {
     Bound b;
     int st = bind(a, b, true);
     if (st != kOk) return st;
@@ -247,25 +275,23 @@ int do_l2(const MegaLaunchArgs& a, hipStream_t s) {
     p.xcd_cuts = p.status + mm::kCutsL2;
     p.queue = at<int>(b, b.L.status) + mm::kQueueL2;
     const int nb = a.hidden / mm::kL2BlockN;
-    // The walk and the one-unit kernel back to back: the device picks one of
-    // them from the routing of this launch (mm::walk_taken).  Tried for 17 to
-    // 128 routed rows per expert on average: below, items of more than 32
-    // rows are rare; above, items of at most 128 rows are (T = 8192); there
-    // the empty launch would only cost time (~5 us for the walk's, ~7 us for
-    // the one-unit kernel's, measured).
-    // Measured on MI355X, walk on vs off: T = 2048 layer 1819-1820 vs
-    // 1846-1847 us (L2 613 vs 645-646); Zipf(1.1) T = 2048 and T = 8192 even
-    // (the one-unit kernel runs them).
+    p.other_queue = at<int>(b, b.L.status) + mm::kQueueL1;
+    p.self_reset = stage == Stage::kAlone;
+    int grid = big_grid(a, b, nb, stage == Stage::kRouted);
+    // The walk is offered for 17 to 128 routed rows per expert on average;
+    // the device takes it if the largest item fits (mm::walk_taken).  Below,
+    // items of more than 32 rows are rare; above, items of at most 128 rows
+    // are (T = 8192).  Measured on MI355X, walk on vs off: T = 2048 layer
+    // 1819-1820 vs 1846-1847 us (L2 613 vs 645-646).
     const int64_t pairs = (int64_t)a.tokens * a.topk;
     if (b.m_tile > 32 && !a.l2_no_walk && !a.mfma_fp8 && pairs > 16LL * a.num_experts &&
         pairs <= 128LL * a.num_experts) {
-        p.walk = 1;
         // at least one workgroup per XCD range (workgroup L walks range L % 8)
-        const int walkers = cu_count() < 8 ? 8 : cu_count();
-        hipLaunchKernelGGL(mm::l2_walk_kernel, dim3(walkers), dim3(mm::kBigThreads), 0, s, p);
+        p.walk = cu_count() < 8 ? 8 : cu_count();
+        if (grid < p.walk) grid = p.walk;
     }
     launch_gemm(kL2Small, a.mfma_fp8 ? mm::l2_big_f8_kernel : mm::l2_big_kernel, b.m_tile, nb,
-                b.L.max_items, s, p);
+                b.L.max_items, grid, s, p);
     return launched(kOk);
 }
 
@@ -299,7 +325,7 @@ int do_reduce(const MegaLaunchArgs& a, hipStream_t s) {
     const bool stream_rows = 2LL * a.tokens * a.topk * a.hidden >= (384LL << 20);
     hipLaunchKernelGGL(stream_rows ? mm::combine_kernel<true> : mm::combine_kernel<false>, grid,
                        dim3(threads), 0, s, at<uint16_t>(b, b.L.l2), at<int>(b, b.L.pair_pos), b.w,
-                       a.topk, a.hidden, a.y, a.y_bf16);
+                       a.topk, a.hidden, a.y, a.y_bf16, at<int>(b, b.L.status) + mm::kQueueL2);
     return launched(kOk);
 }
 
@@ -328,6 +354,7 @@ int do_l1_l2_fused(const MegaLaunchArgs& a, hipStream_t s) {
     p1.out_sf = b.ws + b.L.ffn_sf;
     p1.xcd_cuts = p1.status + mm::kCutsL1;
     p1.queue = at<int>(b, b.L.status) + mm::kQueueL1;
+    p1.self_reset = 1;
     p1.tail_ord = reinterpret_cast<const uint8_t*>(p1.status + mm::kTailOrdL1);
     p2.x = b.ws + b.L.ffn;
     p2.x_sf = a.ffn_ue8m0 ? b.ws + b.L.ffn_sf : nullptr;
@@ -350,6 +377,7 @@ int do_l1_l2_fused(const MegaLaunchArgs& a, hipStream_t s) {
 
 int do_compute(const MegaLaunchArgs& a, hipStream_t s) {
     int st = kOk;
+    const Stage stage = a.skip_prologue ? Stage::kReused : Stage::kRouted;
     if (!a.skip_prologue) {
         st = do_prelude(a, s);
     } else {
@@ -363,10 +391,13 @@ int do_compute(const MegaLaunchArgs& a, hipStream_t s) {
         st = bind(a, b, true);
         if (st == kOk && b.m_tile > 32) return do_l1_l2_fused(a, s);
     }
-    if (st == kOk) st = do_l1(a, s);
-    if (st == kOk) st = do_l2(a, s);
+    if (st == kOk) st = do_l1(a, stage, s);
+    if (st == kOk) st = do_l2(a, stage, s);
     return st;
 }
+
+int do_l1_alone(const MegaLaunchArgs& a, hipStream_t s) { return do_l1(a, Stage::kAlone, s); }
+int do_l2_alone(const MegaLaunchArgs& a, hipStream_t s) { return do_l2(a, Stage::kAlone, s); }
 
 int do_full(const MegaLaunchArgs& a, hipStream_t s) {
     int st = do_compute(a, s);
@@ -518,8 +549,8 @@ MegaLayout layout(int max_tokens, int topk, int num_experts, int hidden, int int
 
 void launch_prelude(const MegaLaunchArgs& a, hipStream_t s) { record(do_prelude(a, s)); }
 void launch_compute(const MegaLaunchArgs& a, hipStream_t s) { record(do_compute(a, s)); }
-void launch_l1(const MegaLaunchArgs& a, hipStream_t s) { record(do_l1(a, s)); }
-void launch_l2(const MegaLaunchArgs& a, hipStream_t s) { record(do_l2(a, s)); }
+void launch_l1(const MegaLaunchArgs& a, hipStream_t s) { record(do_l1_alone(a, s)); }
+void launch_l2(const MegaLaunchArgs& a, hipStream_t s) { record(do_l2_alone(a, s)); }
 void launch_reduce(const MegaLaunchArgs& a, hipStream_t s) { record(do_reduce(a, s)); }
 void launch_full(const MegaLaunchArgs& a, hipStream_t s) { record(do_full(a, s)); }
 void launch_dispatch(const MegaLaunchArgs& a, uint8_t* pool, hipStream_t s) {
@@ -612,7 +643,6 @@ void dump_kernel_resources() {
     print_attr("l2_big_kernel", (const void*)mm::l2_big_kernel);
     print_attr("l1_big_f8_kernel", (const void*)mm::l1_big_f8_kernel);
     print_attr("l2_big_f8_kernel", (const void*)mm::l2_big_f8_kernel);
-    print_attr("l2_walk_kernel", (const void*)mm::l2_walk_kernel);
     print_attr("gemm_fused_kernel", (const void*)mm::gemm_fused_kernel);
     print_attr("combine<cached rows>", (const void*)mm::combine_kernel<false>);
     print_attr("combine<streamed rows>", (const void*)mm::combine_kernel<true>);
@@ -681,8 +711,8 @@ int mm_layout(int max_tokens, int topk, int num_experts, int hidden, int interme
     }
 MM_WRAP(mm_launch_prelude, fp8mega::do_prelude)
 MM_WRAP(mm_launch_compute, fp8mega::do_compute)
-MM_WRAP(mm_launch_l1, fp8mega::do_l1)
-MM_WRAP(mm_launch_l2, fp8mega::do_l2)
+MM_WRAP(mm_launch_l1, fp8mega::do_l1_alone)
+MM_WRAP(mm_launch_l2, fp8mega::do_l2_alone)
 MM_WRAP(mm_launch_reduce, fp8mega::do_reduce)
 MM_WRAP(mm_launch_full, fp8mega::do_full)
 MM_WRAP(mm_launch_full_noalloc, fp8mega::do_full_noalloc)

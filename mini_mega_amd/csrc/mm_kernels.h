@@ -38,9 +38,10 @@ constexpr int kStatusMaxRows = 5;   // status[5]: rows of the largest work item
 constexpr int kCutsL1 = 16;         // status[16..24]: XCD unit ranges of the L1 big GEMM
 constexpr int kCutsL2 = 32;         // status[32..40]: the same for L2
 // Tail queues of the big GEMMs: per XCD a ticket counter over the last
-// kQueueTail units of its range, plus a count of the workgroups that took
-// tickets (status[44..52] for L1, [53..61] for L2; zeroed by the routing
-// scan and again by the last ticket taker of each launch).  L1 always takes
+// kQueueTail units of its range (ranges of more than 2 * kQueueTail units),
+// plus a count of the workgroups that took tickets (status[44..52] for L1,
+// [53..61] for L2; zeroed by the routing scan and again after each GEMM, see
+// gemm_big.hip).  L1 always takes
 // tickets, L2 when its largest item has more than 32 rows (gemm_big.hip:
 // big_unit<true>).  L1's tickets go out costliest unit first: the routing
 // scan writes each tail's order (kTailOrdL1); L2's go out in unit order.
@@ -66,6 +67,9 @@ struct GemmParams {
     const int* status;        // [1] = number of items
     const int* xcd_cuts;      // [9]: XCD x runs big-GEMM units [cuts[x], cuts[x+1])
     int* queue;               // [kQueueInts]: the tail queue of these units
+    int* other_queue;         // the other GEMM's: its launch has ended, this one zeroes it
+    int self_reset;           // 1: the last ticket taker zeroes `queue` (launches not followed by
+                              // the other GEMM's or the combine's)
     const uint8_t* tail_ord;  // [8][kQueueTail]: ticket t of XCD x runs tail unit tail_ord[32x + t]
                               // (null: tail unit t)
     const uint32_t* perm;     // slot -> pair (L1 gathers x rows through it)
@@ -79,8 +83,8 @@ struct GemmParams {
     int ready_target;         // L1 blocks per item (L2 waits for this count)
     int spin_limit;           // L2: polls of a ready counter before giving up
     int* err;                 // status word [0]: kStatusWaitTimeout on give-up
-    // L2 launched as the walk plus the one-unit-per-workgroup kernel: exactly
-    // one of the two runs the units (walk_taken decides from the item size)
+    // L2: workgroups of the walk (0: never); the device runs the units as the
+    // walk or one per workgroup (walk_taken decides from the item size)
     int walk;
 };
 
@@ -102,7 +106,6 @@ __global__ void l1_big_kernel(GemmParams p);
 __global__ void l2_big_kernel(GemmParams p);
 __global__ void l1_big_f8_kernel(GemmParams p);   // MegaLaunchArgs::mfma_fp8
 __global__ void l2_big_f8_kernel(GemmParams p);
-__global__ void l2_walk_kernel(GemmParams p);
 __global__ void gemm_fused_kernel(GemmParams p1, GemmParams p2, int g1);
 
 __global__ void route_hist_kernel(const int64_t*, int, int, int, int*);
@@ -114,7 +117,7 @@ __global__ void dispatch_gather_kernel(const uint8_t*, int, int, const uint32_t*
                                        uint8_t*);
 template <bool kStreamRows>
 __global__ void combine_kernel(const uint16_t*, const int*, const float*, int, int, float*,
-                               uint16_t*);
+                               uint16_t*, int*);
 __global__ void fill_w_lane_kernel(uint8_t*, int, int, uint32_t);
 __global__ void pack_weights_kernel(uint8_t*, const uint8_t*, int, int, int);
 __global__ void pack_weights_ref_kernel(uint8_t*, const uint8_t*, int, int, int);
