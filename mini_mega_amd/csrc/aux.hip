@@ -154,43 +154,11 @@ fill_weights_normal_kernel(uint8_t* __restrict__ w, uint8_t* __restrict__ w_sf, 
     }
 }
 
-// bf16 [rows][cols] -> fp8; sf != null: per-row per-128 UE8M0
-// (utils/math.py:23-47); sf == null: RNE saturating cast (x_fold_body,
-// src/prologue.cuh:103-122).  8 elements per thread, 16 threads per block.
+// bf16 [rows][cols] -> fp8 (quant_act8).
 __global__ void __launch_bounds__(256)
 quant_act_kernel(const uint16_t* __restrict__ x, int rows, int cols, uint8_t* __restrict__ q,
                  uint8_t* __restrict__ sf) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t n8 = (size_t)rows * cols / 8;
-    const bool in = i < n8;
-    float v[8];
-    if (in) {
-        const v4i raw = *reinterpret_cast<const v4i*>(x + i * 8);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            v[2 * c] = bf16_to_f32((uint32_t)raw[c] & 0xFFFFu);
-            v[2 * c + 1] = bf16_to_f32((uint32_t)raw[c] >> 16);
-        }
-    } else {
-#pragma unroll
-        for (int c = 0; c < 8; ++c) v[c] = 0.0f;
-    }
-    float inv = 1.0f;
-    if (sf) {
-        float amax = 0.0f;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) amax = fmaxf(amax, fabsf(v[c]));
-        for (int d = 8; d >= 1; d >>= 1) amax = fmaxf(amax, __shfl_xor(amax, d, 16));
-        const uint32_t sb = block_scale_byte(amax);
-        inv = inv_scale(sb);
-        if (in && (threadIdx.x & 15) == 0) sf[i / 16] = (uint8_t)sb;
-    }
-    if (in) {
-        uint2 o;
-        o.x = pack4_fp8(v[0] * inv, v[1] * inv, v[2] * inv, v[3] * inv);
-        o.y = pack4_fp8(v[4] * inv, v[5] * inv, v[6] * inv, v[7] * inv);
-        *reinterpret_cast<uint2*>(q + i * 8) = o;
-    }
+    quant_act8(x, (size_t)blockIdx.x * blockDim.x + threadIdx.x, (size_t)rows * cols / 8, q, sf);
 }
 
 __global__ void __launch_bounds__(256)

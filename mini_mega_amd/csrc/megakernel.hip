@@ -138,8 +138,24 @@ int do_prelude(const MegaLaunchArgs& a, hipStream_t s) {
     int st = bind(a, b, false);
     if (st != kOk) return st;
     const int E = a.num_experts, P = a.tokens * a.topk;
-    int* status = at<int>(b, b.L.status);   // reset and written by route_scan_kernel
-    fold_x(a, b, s);
+    int* status = at<int>(b, b.L.status);   // reset and written by route_finish
+    const int cap = a.slot_capacity > 0 ? a.slot_capacity : (P > 0 ? P : 1);
+    const int nb1 = a.intermediate / mm::kL1BlockH, nb2 = a.hidden / mm::kL2BlockN;
+    int nbits = 0;
+    while ((1 << nbits) < E) ++nbits;
+    const size_t x8 = a.in_bf16 ? (size_t)a.tokens * a.hidden / 8 : 0;
+    const bool one = P <= mm::kRouteOneP, fold_beside = one && x8 <= mm::kRouteOneFold;
+    if (!fold_beside) fold_x(a, b, s);
+    if (one) {
+        const size_t folds = fold_beside ? (x8 + mm::kScanThreads - 1) / mm::kScanThreads : 0;
+        hipLaunchKernelGGL(mm::route_one_kernel, dim3((unsigned)(1 + folds)),
+                           dim3(mm::kScanThreads), 0, s, a.topk_idx, P, E, nbits, cap, b.m_tile, b.L.max_items, nb1, nb2,
+                           at<int>(b, b.L.counts), at<int>(b, b.L.offsets), at<int>(b, b.L.items),
+                           status, at<uint32_t>(b, b.L.perm), at<int>(b, b.L.pair_pos),
+                           reinterpret_cast<const uint16_t*>(a.self + a.x_off), x8,
+                           b.ws + b.L.xq, a.w1_sf ? b.ws + b.L.xq_sf : nullptr);
+        return launched(kOk);
+    }
     const int chunk = mm::route_chunk(P);
     const int nchunks = P > 0 ? (P + chunk - 1) / chunk : 0;
     int* hist = at<int>(b, b.L.chunk_hist);
@@ -149,14 +165,11 @@ int do_prelude(const MegaLaunchArgs& a, hipStream_t s) {
     if (nchunks > 0 && !fused)
         hipLaunchKernelGGL(mm::route_hist_kernel, dim3(nchunks), dim3(mm::kRouteThreads), 0, s,
                            a.topk_idx, P, E, chunk, hist);
-    const int cap = a.slot_capacity > 0 ? a.slot_capacity : (P > 0 ? P : 1);
     hipLaunchKernelGGL(mm::route_scan_kernel, dim3(1), dim3(mm::kScanThreads), 0, s,
                        fused ? a.topk_idx : nullptr, P, chunk, hist,
-                       nchunks, E, cap, b.m_tile, b.L.max_items, a.intermediate / mm::kL1BlockH,
-                       a.hidden / mm::kL2BlockN, at<int>(b, b.L.counts),
+                       nchunks, E, cap, b.m_tile, b.L.max_items, nb1,
+                       nb2, at<int>(b, b.L.counts),
                        at<int>(b, b.L.offsets), at<int>(b, b.L.items), status);
-    int nbits = 0;
-    while ((1 << nbits) < E) ++nbits;
     if (nchunks > 0)
         hipLaunchKernelGGL(mm::route_scatter_kernel, dim3(nchunks), dim3(mm::kRouteThreads), 0,
                            s, a.topk_idx, P, E, nbits, chunk, hist, at<int>(b, b.L.counts),
@@ -634,6 +647,7 @@ static void print_attr(const char* name, const void* fn) {
 void dump_kernel_resources() {
     print_attr("route_hist", (const void*)mm::route_hist_kernel);
     print_attr("route_scan", (const void*)mm::route_scan_kernel);
+    print_attr("route_one", (const void*)mm::route_one_kernel);
     print_attr("route_scatter", (const void*)mm::route_scatter_kernel);
     print_attr("l1_kernel<1>", (const void*)mm::l1_kernel<1>);
     print_attr("l1_kernel<2>", (const void*)mm::l1_kernel<2>);

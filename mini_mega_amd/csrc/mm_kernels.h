@@ -22,6 +22,17 @@ inline int route_chunk(int P) { return P <= kRouteSmallP ? kRouteChunkSmall : kR
 // when they fit: nchunks * E <= kFusedHist counters.
 constexpr int kFusedHist = 8192;
 
+// One workgroup does the whole routing (route_one_kernel) up to this many
+// pairs and segment counters (segments of 64 pairs x experts, 16 bits each).
+constexpr int kRouteOneRounds = 4;
+constexpr int kRouteOneP = kRouteOneRounds * kScanThreads;
+constexpr int kRouteOneSegs = 65536;
+// Groups of 8 activations that route_one_kernel folds beside the routing: two
+// workgroups per CU (its LDS allows one at a time); a larger fold keeps its own
+// launch.
+constexpr size_t kRouteOneFold = 512 * kScanThreads;
+static_assert(kRouteOneP / 64 * kMaxExperts <= kRouteOneSegs, "the segment counters fit");
+
 constexpr int kGemmThreads = 256;   // 4 waves per workgroup (decode-shaped GEMMs)
 constexpr int kBigThreads = 512;    // 8 waves per workgroup, two per SIMD (large-M GEMMs)
 constexpr int kBigMaxTiles = 16;    // large-M GEMMs: up to 16 token tiles (256 rows) per item
@@ -111,6 +122,9 @@ __global__ void gemm_fused_kernel(GemmParams p1, GemmParams p2, int g1);
 __global__ void route_hist_kernel(const int64_t*, int, int, int, int*);
 __global__ void route_scan_kernel(const int64_t*, int, int, int*, int, int, int, int, int, int, int,
                                   int*, int*, int*, int*);
+__global__ void route_one_kernel(const int64_t*, int, int, int, int, int, int, int, int, int*, int*,
+                                 int*, int*, uint32_t*, int*, const uint16_t*, size_t, uint8_t*,
+                                 uint8_t*);
 __global__ void route_scatter_kernel(const int64_t*, int, int, int, int, const int*, const int*,
                                      const int*, uint32_t*, int*);
 __global__ void dispatch_gather_kernel(const uint8_t*, int, int, const uint32_t*, const int*,

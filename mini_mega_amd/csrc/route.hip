@@ -2,8 +2,9 @@
 // the reference's EP dispatch metadata: route_build_body, src/prologue.cuh:
 // 126-226; publish_counts_body :230-256; task_setup_body :269-498).
 //
-// Three stream-ordered kernels over P = tokens * topk (token, k) pairs (two
-// for small P, where route_scan builds the histograms itself):
+// P = tokens * topk (token, k) pairs.  Up to kRouteOneP pairs one workgroup does
+// it all (route_one); above, three stream-ordered kernels (two where route_scan
+// builds the histograms itself):
 //   1. route_hist:    per chunk of pairs, an LDS histogram over experts.
 //   2. route_scan:    one workgroup; per expert the exclusive prefix over chunks,
 //                     the capped count, the exclusive prefix over experts
@@ -38,31 +39,224 @@ route_hist_kernel(const int64_t* __restrict__ topk_idx, int P, int E, int chunk,
         chunk_hist[(size_t)blockIdx.x * E + i] = hist[i];
 }
 
-// Block-wide exclusive scan of one int per thread (blockDim = kScanThreads).
-__device__ int block_exclusive_scan(int v, int* smem, int* total) {
+// Block-wide exclusive scan of one int4 per thread, component by component
+// (blockDim = kScanThreads); *total: the sums.
+__device__ int4 block_exclusive_scan4(int4 v, int4* smem, int4* total) {
+    constexpr int kWaves = kScanThreads / 64;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int x = v;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int y = __shfl_up(x, d, 64);
-        if (lane >= d) x += y;
-    }
+    auto wave_scan = [&](int4 x, int n) {   // inclusive, over the first n lanes
+        for (int d = 1; d < n; d <<= 1) {
+            const int4 y = make_int4(__shfl_up(x.x, d, 64), __shfl_up(x.y, d, 64),
+                                     __shfl_up(x.z, d, 64), __shfl_up(x.w, d, 64));
+            if (lane >= d) {
+                x.x += y.x;
+                x.y += y.y;
+                x.z += y.z;
+                x.w += y.w;
+            }
+        }
+        return x;
+    };
+    const int4 x = wave_scan(v, 64);
     if (lane == 63) smem[wave] = x;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        int run = 0;
-        for (int w = 0; w < kScanThreads / 64; ++w) {
-            const int t = smem[w];
-            smem[w] = run;
-            run += t;
-        }
-        smem[kScanThreads / 64] = run;
+    const int4 t = wave_scan(smem[lane & (kWaves - 1)], kWaves);   // the waves' running sums
+    const int prev = wave > 0 ? wave - 1 : 0, on = wave > 0;
+    *total = make_int4(__shfl(t.x, kWaves - 1, 64), __shfl(t.y, kWaves - 1, 64),
+                       __shfl(t.z, kWaves - 1, 64), __shfl(t.w, kWaves - 1, 64));
+    return make_int4(on * __shfl(t.x, prev, 64) + x.x - v.x, on * __shfl(t.y, prev, 64) + x.y - v.y,
+                     on * __shfl(t.z, prev, 64) + x.z - v.z, on * __shfl(t.w, prev, 64) + x.w - v.w);
+}
+
+// LDS of route_finish.
+struct RouteSmem {
+    int4 waves[kScanThreads / 64];
+    int cuts[9];                       // the L1 XCD unit ranges
+    int rows;                          // rows of the largest work item
+    int ioff[kMaxExperts + 1];         // first item of each expert (+ the item count)
+    int cnt[kMaxExperts];              // routed rows of each expert
+    int off[kMaxExperts];              // first slot of each expert
+    int cost[kMaxExperts];             // modelled cost of the experts before it
+    uint8_t tnt[8][kQueueTail];        // token tiles of L1's tail units
+};
+
+struct RouteOut {
+    int* counts;
+    int* offsets;
+    int* items;
+    int* status;
+};
+
+// Everything the routing derives from the experts' pair counts: called by all
+// kScanThreads threads of one workgroup, thread e holding expert e's pairs
+// `run` (E <= kMaxExperts = kScanThreads).  The four running sums it needs
+// (pairs, routed rows, items, modelled cost) follow from `run` alone, so one
+// scan makes them all (measured on MI355X at T = 1, one scan each, thread 0
+// summing the waves, and a 64-bit division for each XCD cut: routing 11.4 us in
+// two launches, 6.5 in one with this).
+__device__ void route_finish(RouteSmem& sh, int run, int P, int E, int cap, int m_tile,
+                             int max_items, int nb1, int nb2, const RouteOut& o) {
+    const int e = threadIdx.x;
+    const int cnt = min(run, cap);   // 0 for e >= E
+    if (e < E) {
+        o.counts[e] = cnt;
+        sh.cnt[e] = cnt;
     }
+    // the status word of this launch (only this kernel sets its error bits;
+    // thread 0 clears it before its own atomicOr below)
+    if (e == 0) {
+        o.status[0] = 0;
+        sh.rows = 0;
+    }
+    // Work items: the expert's rows split evenly into ceil(cnt / m_tile)
+    // items of at most m_tile rows (no item re-streams the expert's weights
+    // for a small remainder).  The items of one expert then have equal token
+    // tile counts, so the units that read one weight block run in lockstep
+    // and all but the first take it from L2.  (Measured on MI355X at T =
+    // 8192: splitting at 16-row multiples instead ran 2% less MFMA work but
+    // its unequal items drifted apart; L1 fetched 9.30 vs 7.33 GB and the
+    // layer took 4908-4943 vs 4841-4854 us.)  Record: (expert, first slot,
+    // end slot, index within the expert | item count of the expert << 16),
+    // the slots absolute (the expert's offset included), so that a GEMM unit
+    // needs no offsets[] load after its item.
+    const int nm = (cnt + m_tile - 1) / m_tile;
+    const int sz = nm > 0 ? (cnt + nm - 1) / nm : 0;
+    // XCD ranges of the big GEMMs' units (nb blocks per item; an expert's
+    // nb * nm units are contiguous in the kernels' numbering).  Modelled cost
+    // of one of the expert's units per k-step, in token-tile MFMA times:
+    // max(9, 2 + token tiles of its largest item) -- the fixed per-step work
+    // (barrier, conversions, operand reads) is worth ~2 token tiles and the
+    // weight stream at the full-chip HBM rate ~9 (measured on MI355X: a
+    // k-step costs ~0.33 us + 0.137 us per token tile without weight loads,
+    // and a weight block's k-step streams in ~1.23 us).  XCD x starts where
+    // the running cost crosses x/8 of the total (the same expert for L1 and
+    // L2, whose costs differ by the factor nb); each range is then clamped to
+    // its share of the grid, nb * max_items + 8 workgroups.
+    const int uc = max(9, 2 + min((sz + 15) >> 4, kBigMaxTiles));
+    const int w = nm * uc;
+    __syncthreads();   // sh.rows
+    if (sz > 0) atomicMax(&sh.rows, sz);   // ordered before the read by the scan's barrier
+    int4 tot;
+    const int4 pre = block_exclusive_scan4(make_int4(run, cnt, nm, w), sh.waves, &tot);
+    // valid: pairs with an id in [0, E) before the slot cap (the rest of P had
+    // ids outside [0, E))
+    const int off = pre.y, ioff = pre.z, wpre = pre.w;
+    const int valid = tot.x, slots = tot.y, nitems = tot.z, wtot = tot.w;
+    if (e < E) {
+        o.offsets[e] = off;
+        sh.off[e] = off;
+    }
+    if (e == 0) o.offsets[E] = slots;
+    for (int j = 0; j < nm; ++j) {
+        const int it = ioff + j;
+        if (it < max_items) {
+            const int m0 = j * sz;
+            reinterpret_cast<int4*>(o.items)[it] =
+                make_int4(e, off + m0, off + min(cnt, m0 + sz), j | (nm << 16));
+        }
+    }
+    if (threadIdx.x < 2 * kQueueInts) o.status[kQueueL1 + threadIdx.x] = 0;   // tail queues
+    // per-item L1 ready counters of the fused L1 -> L2 launch (after the table)
+    for (int i = threadIdx.x; i < max_items; i += kScanThreads) o.items[4 * max_items + i] = 0;
+    if (e == 0) {
+        o.status[1] = min(nitems, max_items);
+        o.status[2] = slots;
+        o.status[3] = valid - slots;   // pairs dropped by the slot capacity
+        o.status[4] = P - valid;       // pairs whose expert id is outside [0, E)
+        o.status[kStatusMaxRows] = sh.rows;
+        if (nitems > max_items) atomicOr(&o.status[0], kStatusItemOverflow);
+    }
+    if (e < E) {
+        sh.cost[e] = wpre;
+        sh.ioff[e] = ioff;
+    }
+    if (e == 0) sh.ioff[E] = nitems;
     __syncthreads();
-    const int r = smem[wave] + x - v;
-    *total = smem[kScanThreads / 64];
-    __syncthreads();
-    return r;
+    // One thread per cut (XCD x of L1: threads 0-7, of L2: 8-15) finds the
+    // expert that its target cost falls in: the last one whose running cost is
+    // not above it (never an empty one: the next expert's is the same).
+    if (e < 16) {
+        const int g = e >> 3, x = e & 7, nb = g == 0 ? nb1 : nb2;
+        const int n = min(nitems, max_items), units = nb * n, share = (nb * max_items + 8) / 8;
+        // a target past the last complete expert (item overflow) cuts at the end
+        int v = units;
+        if (nitems <= max_items && n > 0) {
+            const int64_t t = (int64_t)wtot * nb * x / 8;
+            int lo = 0, hi = E - 1;
+            while (lo < hi) {
+                const int m = (lo + hi + 1) >> 1;
+                if ((int64_t)sh.cost[m] * nb <= t) lo = m; else hi = m - 1;
+            }
+            const int c = sh.cnt[lo], cn = (c + m_tile - 1) / m_tile;
+            const int cz = (c + cn - 1) / cn;
+            const int ucl = max(9, 2 + min((cz + 15) >> 4, kBigMaxTiles));
+            // below nb * nm * ucl of one expert: 32 bits
+            v = nb * sh.ioff[lo] + (int)((uint32_t)(t - (int64_t)sh.cost[lo] * nb) / (uint32_t)ucl);
+        }
+        int* cuts = o.status + (g == 0 ? kCutsL1 : kCutsL2);
+        int prev = 0, mine = 0;
+#pragma unroll
+        for (int y = 1; y < 8; ++y) {
+            int c = __shfl(v, 8 * g + y, 64);
+            c = min(max(c, prev), prev + share);
+            c = max(c, units - (8 - y) * share);
+            if (y == x) mine = c;
+            prev = c;
+        }
+        cuts[x] = mine;
+        if (x == 0) cuts[8] = units;
+        if (g == 0) {
+            sh.cuts[x] = mine;
+            if (x == 0) sh.cuts[8] = units;
+        }
+    }
+    // Ticket order of L1's tail queues (the last t = min(range, kQueueTail)
+    // units of each XCD range): costliest unit first, i.e. by the token tiles
+    // of its item, descending, ties in unit order, so that heavy units do not
+    // start after light ones at the end of the kernel.  Tail unit i of XCD x
+    // is unit cuts[x + 1] - t + i; L1 runs ticket k as tail unit order[k]
+    // (gemm_big.hip: claim_tail_unit).  One thread per tail slot finds its
+    // unit's expert by binary search over the item offsets.  Only when some
+    // item holds more than kTailOrderRows rows (skewed routing, T = 8192):
+    // below, the units differ by a few token tiles at most, and the order is
+    // the identity.  (Measured on MI355X: a loop over the 8 tails in every
+    // expert thread added 10.6 us to this one-workgroup kernel; L2's tails
+    // gained nothing from the order and keep ticket order.)
+    uint8_t* order = reinterpret_cast<uint8_t*>(o.status + kTailOrdL1);
+    __syncthreads();   // sh.cuts, and sh.rows of every expert
+    if (sh.rows > kTailOrderRows) {   // uniform over the workgroup
+        if (threadIdx.x < 8 * kQueueTail) {
+            const int x = threadIdx.x / kQueueTail, i = threadIdx.x % kQueueTail;
+            const int lo = sh.cuts[x], hi = sh.cuts[x + 1], t = min(hi - lo, kQueueTail);
+            if (i < t) {
+                const int u = hi - t + i, im = u / nb1;
+                int a = 0, b = E - 1;   // the last expert whose first item is <= im
+                while (a < b) {
+                    const int m = (a + b + 1) >> 1;
+                    if (sh.ioff[m] <= im) a = m; else b = m - 1;
+                }
+                const int n = max(sh.ioff[a + 1] - sh.ioff[a], 1), c = sh.cnt[a];
+                const int z = (c + n - 1) / n, j = (u - nb1 * sh.ioff[a]) % n;
+                sh.tnt[x][i] = (uint8_t)min((min(c, (j + 1) * z) - j * z + 15) >> 4, kBigMaxTiles);
+            }
+        }
+        __syncthreads();
+        if (threadIdx.x < 8 * kQueueTail) {
+            const int x = threadIdx.x / kQueueTail, i = threadIdx.x % kQueueTail;
+            const int t = min(sh.cuts[x + 1] - sh.cuts[x], kQueueTail);
+            if (i < t) {
+                const int v = sh.tnt[x][i];
+                int r = 0;
+                for (int k = 0; k < t; ++k) {
+                    const int w = sh.tnt[x][k];
+                    r += (w > v) || (w == v && k < i);
+                }
+                order[kQueueTail * x + r] = (uint8_t)i;
+            }
+        }
+    } else if (threadIdx.x < 8 * kQueueTail) {
+        order[threadIdx.x] = (uint8_t)(threadIdx.x % kQueueTail);
+    }
 }
 
 __global__ void __launch_bounds__(kScanThreads)
@@ -70,20 +264,8 @@ route_scan_kernel(const int64_t* __restrict__ topk_idx, int P, int chunk,
                   int* __restrict__ chunk_hist, int nchunks, int E, int cap, int m_tile,
                   int max_items, int nb1, int nb2, int* __restrict__ counts,
                   int* __restrict__ offsets, int* __restrict__ items, int* __restrict__ status) {
-    __shared__ int smem[kScanThreads / 64 + 1];
-    __shared__ int cut_s[2][8];
+    __shared__ RouteSmem sh;
     __shared__ int lh[kFusedHist];   // [chunk][expert] when topk_idx is given
-    __shared__ int s_rows;           // rows of the largest work item
-    __shared__ int cuts_sh[9];       // the L1 XCD unit ranges
-    __shared__ int s_ioff[kMaxExperts + 1];     // first item of each expert (+ the item count)
-    __shared__ int s_cnt[kMaxExperts];          // routed rows of each expert
-    __shared__ uint8_t tnt[8][kQueueTail];      // token tiles of L1's tail units
-    // the status word of this launch (only this kernel sets its error bits;
-    // thread 0 clears it before its own atomicOr below)
-    if (threadIdx.x == 0) {
-        status[0] = 0;
-        s_rows = 0;
-    }
     // Small launches (topk_idx given, nchunks * E <= kFusedHist): the chunk
     // histograms of route_hist_kernel, built here in LDS, 8 pairs' loads in
     // flight per thread.
@@ -108,7 +290,7 @@ route_scan_kernel(const int64_t* __restrict__ topk_idx, int P, int chunk,
     }
     // E <= kMaxExperts = kScanThreads: one expert per thread.
     const int e = threadIdx.x;
-    int cnt = 0, run = 0;
+    int run = 0;
     if (e < E) {
         // exclusive prefix over chunks (uncapped rank base), 8 chunks' loads
         // in flight at a time
@@ -126,151 +308,97 @@ route_scan_kernel(const int64_t* __restrict__ topk_idx, int P, int chunk,
                     run += h[u];
                 }
         }
-        cnt = min(run, cap);
-        counts[e] = cnt;
     }
-    // pairs with an id in [0, E) before the slot cap (the rest of P had ids
-    // outside [0, E))
-    int valid = 0;
-    (void)block_exclusive_scan(run, smem, &valid);
-    int slots = 0;
-    const int off = block_exclusive_scan(cnt, smem, &slots);
-    if (e < E) offsets[e] = off;
-    if (threadIdx.x == 0) offsets[E] = slots;
-    // Work items: the expert's rows split evenly into ceil(cnt / m_tile)
-    // items of at most m_tile rows (no item re-streams the expert's weights
-    // for a small remainder).  The items of one expert then have equal token
-    // tile counts, so the units that read one weight block run in lockstep
-    // and all but the first take it from L2.  (Measured on MI355X at T =
-    // 8192: splitting at 16-row multiples instead ran 2% less MFMA work but
-    // its unequal items drifted apart; L1 fetched 9.30 vs 7.33 GB and the
-    // layer took 4908-4943 vs 4841-4854 us.)  Record: (expert, first slot,
-    // end slot, index within the expert | item count of the expert << 16),
-    // the slots absolute (the expert's offset included), so that a GEMM unit
-    // needs no offsets[] load after its item.
-    const int nm = (cnt + m_tile - 1) / m_tile;
-    const int sz = nm > 0 ? (cnt + nm - 1) / nm : 0;
-    if (sz > 0) atomicMax(&s_rows, sz);   // ordered before the read by the scan's barriers
-    int nitems = 0;
-    const int ioff = block_exclusive_scan(nm, smem, &nitems);
-    for (int j = 0; j < nm; ++j) {
-        const int it = ioff + j;
-        if (it < max_items) {
-            const int m0 = j * sz;
-            reinterpret_cast<int4*>(items)[it] =
-                make_int4(e, off + m0, off + min(cnt, m0 + sz), j | (nm << 16));
+    route_finish(sh, run, P, E, cap, m_tile, max_items, nb1, nb2,
+                 RouteOut{counts, offsets, items, status});
+}
+
+// The whole routing in one workgroup, for at most kRouteOneSegs segments x
+// experts counters and kRouteOneRounds rounds: a segment is 64 consecutive
+// pairs, one per lane of a wave.  Every wave ranks its pairs within the
+// segment (ballots over the expert-id bits) and counts them per expert in
+// LDS; thread e then runs over the segments for expert e's running counts, and
+// a pair's slot is its expert's offset + the count before its segment + its
+// rank.  The pairs are read once and stay in registers.
+// Latency-bound: one launch instead of two or three (measured on MI355X, all
+// routing kernels, E = 256: T = 1 11.4 -> 6.5 us, T = 13 11.9 -> 7.3, T = 512
+// 15.6 -> 14.2).  Workgroups after the first fold bf16 activations (x8 groups
+// of 8 values), a launch of its own otherwise.
+__global__ void __launch_bounds__(kScanThreads)
+route_one_kernel(const int64_t* __restrict__ topk_idx, int P, int E, int nbits, int cap,
+                 int m_tile, int max_items, int nb1, int nb2, int* __restrict__ counts,
+                 int* __restrict__ offsets, int* __restrict__ items, int* __restrict__ status,
+                 uint32_t* __restrict__ perm, int* __restrict__ pair_pos,
+                 const uint16_t* __restrict__ x, size_t x8, uint8_t* __restrict__ xq,
+                 uint8_t* __restrict__ xq_sf) {
+    if (blockIdx.x > 0) {   // the fold of bf16 activations, next to the routing
+        quant_act8(x, (size_t)(blockIdx.x - 1) * kScanThreads + threadIdx.x, x8, xq, xq_sf);
+        return;
+    }
+    __shared__ RouteSmem sh;
+    __shared__ __align__(16) uint16_t seg[kRouteOneSegs];   // [segment][expert]
+    constexpr int kWaves = kScanThreads / 64;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int nseg = (P + 63) >> 6;
+    int64_t ev[kRouteOneRounds];
+#pragma unroll
+    for (int r = 0; r < kRouteOneRounds; ++r) {
+        const int p = r * kScanThreads + threadIdx.x;
+        ev[r] = p < P ? topk_idx[p] : -1;
+    }
+    for (int i = threadIdx.x * 8; i < nseg * E; i += kScanThreads * 8)   // E * nseg <= kRouteOneSegs
+        *reinterpret_cast<v4i*>(&seg[i]) = v4i{0, 0, 0, 0};
+    __syncthreads();
+    const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    int rank[kRouteOneRounds];
+#pragma unroll
+    for (int r = 0; r < kRouteOneRounds; ++r) {
+        if (r * kScanThreads + wave * 64 >= P) break;   // uniform over the wave
+        const bool ok = ev[r] >= 0 && ev[r] < E;
+        const int e = ok ? (int)ev[r] : 0;
+        // lanes holding the same expert id: AND of per-bit ballots
+        uint64_t m = __ballot(ok);
+        for (int b = 0; b < nbits; ++b) {
+            const uint64_t bb = __ballot(ok && ((e >> b) & 1));
+            m &= ((e >> b) & 1) ? bb : ~bb;
         }
-    }
-    if (threadIdx.x < 2 * kQueueInts) status[kQueueL1 + threadIdx.x] = 0;   // tail queues
-    // per-item L1 ready counters of the fused L1 -> L2 launch (after the table)
-    for (int i = threadIdx.x; i < max_items; i += kScanThreads) items[4 * max_items + i] = 0;
-    if (threadIdx.x == 0) {
-        status[1] = min(nitems, max_items);
-        status[2] = slots;
-        status[3] = valid - slots;   // pairs dropped by the slot capacity
-        status[4] = P - valid;       // pairs whose expert id is outside [0, E)
-        status[kStatusMaxRows] = s_rows;
-        if (nitems > max_items) atomicOr(&status[0], kStatusItemOverflow);
-    }
-    // XCD ranges of the big GEMMs' units (nb blocks per item; an expert's
-    // nb * nm units are contiguous in the kernels' numbering).  Modelled cost
-    // of one of the expert's units per k-step, in token-tile MFMA times:
-    // max(9, 2 + token tiles of its largest item) -- the fixed per-step work
-    // (barrier, conversions, operand reads) is worth ~2 token tiles and the
-    // weight stream at the full-chip HBM rate ~9 (measured on MI355X: a
-    // k-step costs ~0.33 us + 0.137 us per token tile without weight loads,
-    // and a weight block's k-step streams in ~1.23 us).  XCD x starts where
-    // the running cost crosses x/8 of the total (the same expert for L1 and
-    // L2, whose costs differ by the factor nb); each range is then clamped to
-    // its share of the grid, nb * max_items + 8 workgroups.
-    const int uc = max(9, 2 + min((sz + 15) >> 4, kBigMaxTiles));
-    const int w = nm * uc;
-    int wtot = 0;
-    const int wpre = block_exclusive_scan(w, smem, &wtot);
-    if (nm > 0 && ioff + nm <= max_items) {
-        for (int x = 1; x < 8; ++x) {
-            const int64_t t1 = (int64_t)wtot * nb1 * x / 8, t2 = (int64_t)wtot * nb2 * x / 8;
-            const int64_t lo1 = (int64_t)wpre * nb1, lo2 = (int64_t)wpre * nb2;
-            if (t1 >= lo1 && t1 < lo1 + (int64_t)w * nb1)
-                cut_s[0][x] = nb1 * ioff + (int)((t1 - lo1) / uc);
-            if (t2 >= lo2 && t2 < lo2 + (int64_t)w * nb2)
-                cut_s[1][x] = nb2 * ioff + (int)((t2 - lo2) / uc);
-        }
+        rank[r] = __popcll(m & lt_mask);
+        if (ok && rank[r] == 0) seg[(r * kWaves + wave) * E + e] = (uint16_t)__popcll(m);
     }
     __syncthreads();
-    if (threadIdx.x < 2) {
-        const int nb = threadIdx.x == 0 ? nb1 : nb2;
-        const int n = min(nitems, max_items), units = nb * n, cap = (nb * max_items + 8) / 8;
-        int* cuts = status + (threadIdx.x == 0 ? kCutsL1 : kCutsL2);
-        int prev = 0;
-        cuts[0] = 0;
-        for (int x = 1; x < 8; ++x) {
-            // a target past the last complete expert (item overflow) cuts at the end
-            int v = nitems <= max_items && n > 0 ? cut_s[threadIdx.x][x] : units;
-            v = min(max(v, prev), prev + cap);
-            v = max(v, units - (8 - x) * cap);
-            cuts[x] = v;
-            if (threadIdx.x == 0) cuts_sh[x] = v;
-            prev = v;
-        }
-        cuts[8] = units;
-        if (threadIdx.x == 0) {
-            cuts_sh[0] = 0;
-            cuts_sh[8] = units;
+    int run = 0;
+    if ((int)threadIdx.x < E) {
+        // 8 segments' counts in flight at a time
+        for (int s0 = 0; s0 < nseg; s0 += 8) {
+            int h[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                h[u] = s0 + u < nseg ? seg[(s0 + u) * E + threadIdx.x] : 0;
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (s0 + u < nseg) {
+                    seg[(s0 + u) * E + threadIdx.x] = (uint16_t)run;
+                    run += h[u];
+                }
         }
     }
-    // Ticket order of L1's tail queues (the last t = min(range, kQueueTail)
-    // units of each XCD range): costliest unit first, i.e. by the token tiles
-    // of its item, descending, ties in unit order, so that heavy units do not
-    // start after light ones at the end of the kernel.  Tail unit i of XCD x
-    // is unit cuts[x + 1] - t + i; L1 runs ticket k as tail unit order[k]
-    // (gemm_big.hip: claim_tail_unit).  One thread per tail slot finds its
-    // unit's expert by binary search over the item offsets.  Only when some
-    // item holds more than kTailOrderRows rows (skewed routing, T = 8192):
-    // below, the units differ by a few token tiles at most, and the order is
-    // the identity.  (Measured on MI355X: a loop over the 8 tails in every
-    // expert thread added 10.6 us to this one-workgroup kernel; L2's tails
-    // gained nothing from the order and keep ticket order.)
-    uint8_t* order = reinterpret_cast<uint8_t*>(status + kTailOrdL1);
-    __syncthreads();   // cuts_sh, and s_rows of every expert
-    if (s_rows > kTailOrderRows) {   // uniform over the workgroup
-        if (e < E) {
-            s_ioff[e] = ioff;
-            s_cnt[e] = cnt;
-        }
-        if (threadIdx.x == 0) s_ioff[E] = nitems;
-        __syncthreads();
-        if (threadIdx.x < 8 * kQueueTail) {
-            const int x = threadIdx.x / kQueueTail, i = threadIdx.x % kQueueTail;
-            const int lo = cuts_sh[x], hi = cuts_sh[x + 1], t = min(hi - lo, kQueueTail);
-            if (i < t) {
-                const int u = hi - t + i, im = u / nb1;
-                int a = 0, b = E - 1;   // the last expert whose first item is <= im
-                while (a < b) {
-                    const int m = (a + b + 1) >> 1;
-                    if (s_ioff[m] <= im) a = m; else b = m - 1;
-                }
-                const int n = max(s_ioff[a + 1] - s_ioff[a], 1), c = s_cnt[a];
-                const int z = (c + n - 1) / n, j = (u - nb1 * s_ioff[a]) % n;
-                tnt[x][i] = (uint8_t)min((min(c, (j + 1) * z) - j * z + 15) >> 4, kBigMaxTiles);
+    route_finish(sh, run, P, E, cap, m_tile, max_items, nb1, nb2,
+                 RouteOut{counts, offsets, items, status});
+    // sh.cnt, sh.off and seg were written before route_finish's barriers
+#pragma unroll
+    for (int r = 0; r < kRouteOneRounds; ++r) {
+        const int p = r * kScanThreads + threadIdx.x;
+        if (p >= P) break;
+        int pos = -1;
+        if (ev[r] >= 0 && ev[r] < E) {
+            const int e = (int)ev[r];
+            const int k = seg[(r * kWaves + wave) * E + e] + rank[r];
+            if (k < sh.cnt[e]) {
+                pos = sh.off[e] + k;
+                perm[pos] = (uint32_t)p;
             }
         }
-        __syncthreads();
-        if (threadIdx.x < 8 * kQueueTail) {
-            const int x = threadIdx.x / kQueueTail, i = threadIdx.x % kQueueTail;
-            const int t = min(cuts_sh[x + 1] - cuts_sh[x], kQueueTail);
-            if (i < t) {
-                const int v = tnt[x][i];
-                int r = 0;
-                for (int k = 0; k < t; ++k) {
-                    const int w = tnt[x][k];
-                    r += (w > v) || (w == v && k < i);
-                }
-                order[kQueueTail * x + r] = (uint8_t)i;
-            }
-        }
-    } else if (threadIdx.x < 8 * kQueueTail) {
-        order[threadIdx.x] = (uint8_t)(threadIdx.x % kQueueTail);
+        pair_pos[p] = pos;
     }
 }
 

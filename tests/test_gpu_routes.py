@@ -1,0 +1,60 @@
+"""GPU tests of the one-workgroup routing at the edges of its segments and
+limits, and of the activation fold beside it, against the oracle's routing and
+the fold's own kernel."""
+import dataclasses
+
+import numpy as np
+import pytest
+import torch
+
+import mini_mega_amd as mm
+from mini_mega_amd import inputs
+
+import moe_case as mc
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+# pairs around a segment (64), a round (1024) and the last size of the one-
+# workgroup routing (4096), with few experts and the most
+@pytest.mark.parametrize("T,K,E", [(1, 1, 1), (63, 1, 8), (64, 1, 8), (65, 1, 1024), (1023, 1, 256),
+                                   (1025, 1, 1024), (819, 5, 128), (4095, 1, 1024), (512, 8, 256),
+                                   (4097, 1, 1024)])
+def test_routing_around_the_one_workgroup_limits(T, K, E):
+    rng = np.random.default_rng(T * 31 + E)
+    idx = rng.integers(0, E, size=(T, K)).astype(np.int64)
+    idx[rng.random((T, K)) < 0.3] = E // 2          # a hot expert, repeats within a wave
+    bad = rng.random((T, K)) < 0.05
+    idx[bad] = rng.choice([-1, E, E + 7, 1 << 40], size=int(bad.sum()))
+    for cap in (0, max(1, T * K // (2 * E))):
+        c = mc.normal_case(E, K, 256, 128, T, seed=3, scaled=False, idx=idx,
+                           wts=np.full((T, K), 1.0 / K, np.float32))
+        c = dataclasses.replace(c, cap=cap)
+        r = mc.run_layer(c)
+        mc.check_routing(c, r)
+        mc.check_reduce(c, r)
+
+
+# the fold runs beside the routing up to 524288 groups of 8 values (T = 512 at
+# H = 8192), in a launch of its own above; T = 37: a partly filled workgroup
+@pytest.mark.parametrize("T,H,scaled", [(37, 256, True), (512, 8192, True), (513, 8192, False)])
+def test_fold_beside_the_routing(T, H, scaled):
+    E, K, I = 4, 2, 128
+    xb, xq, xsf = inputs.make_x(T, H, seed=T, scaled=scaled)
+    (w1, s1), (w2, s2) = inputs.make_weights_normal(E, H, I, seed=6)
+    idx, wts = inputs.route(T, E, K, seed=7)
+    buf = mm.get_symm_buffer_for_mega_moe(None, E, T, K, H, I, mma_type="bf16xfp8")
+    buf.x[:T].copy_(xb)
+    buf.topk_idx[:T].copy_(torch.from_numpy(idx))
+    buf.topk_weights[:T].copy_(torch.from_numpy(wts))
+    y = torch.empty((T, H), dtype=torch.bfloat16, device="cuda")
+    mm.bf16_fp8_mega_moe(y, (w1, s1) if scaled else w1, (w2, s2) if scaled else w2, buf)
+    torch.cuda.synchronize()
+    L = buf.layout
+    assert torch.equal(buf.workspace[L.xq:L.xq + T * H].view(T, H), xq)
+    if scaled:
+        assert torch.equal(buf.workspace[L.xq_sf:L.xq_sf + T * (H // 128)].view(T, H // 128), xsf)
+    counts, offsets, perm, pair_pos = orc.route(idx, E, None)
+    assert np.array_equal(buf.counts().cpu().numpy(), counts)
+    assert np.array_equal(buf.pair_pos(T).cpu().numpy().ravel(), np.asarray(pair_pos).ravel())
