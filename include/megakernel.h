@@ -225,6 +225,11 @@ int read_status(const MegaLaunchArgs& a, int32_t* out, int n, hipStream_t stream
 // Logical row-major [n_mats][n_rows][k_cols] fp8 -> tile layout.
 void pack_weights(uint8_t* dst, const uint8_t* src, int n_mats, int n_rows,
                   int k_cols, hipStream_t stream);
+// The same for W1 given as [gate; up] halves: the rows are also put in the
+// paired order, gate and up alternating in blocks of `pair` rows (n_rows %
+// (2 * pair) == 0).
+void pack_weights_paired(uint8_t* dst, const uint8_t* src, int n_mats, int n_rows,
+                         int k_cols, int pair, hipStream_t stream);
 // The reference's packed on-device weights (lane-tile layout: fill_w_lane
 // bytes, src/megakernel.cu:66-105, closed form src/bench_check.cuh:268-272;
 // the output of its transform_weights_for_mega_moe,
@@ -293,6 +298,8 @@ int mm_fill_weights_lane(uint8_t* w, int n_rows, int k_cols, unsigned seed,
                          void* stream);
 int mm_pack_weights(uint8_t* dst, const uint8_t* src, int n_mats, int n_rows,
                     int k_cols, void* stream);
+int mm_pack_weights_paired(uint8_t* dst, const uint8_t* src, int n_mats,
+                           int n_rows, int k_cols, int pair, void* stream);
 int mm_pack_weights_from_reference(uint8_t* dst, const uint8_t* src, int n_mats,
                                    int n_rows, int k_cols, void* stream);
 int mm_fill_weights_normal(uint8_t* w, uint8_t* w_sf, int n_mats, int n_rows,

@@ -67,7 +67,7 @@ EXPORTS = (
     "mm_launch_compute", "mm_launch_l1", "mm_launch_l2", "mm_launch_reduce", "mm_launch_full",
     "mm_launch_full_noalloc", "mm_noalloc_scratch_bytes",
     "mm_launch_empty", "mm_launch_dispatch", "mm_read_status", "mm_fill_weights_lane", "mm_pack_weights",
-    "mm_pack_weights_from_reference",
+    "mm_pack_weights_paired", "mm_pack_weights_from_reference",
     "mm_fill_weights_normal", "mm_quant_act", "mm_selftest_convert", "mm_dump_kernel_resources",
     "mm_probe_mfma_dot", "mm_probe_l2_rows", "mm_probe_stream_read", "mm_probe_mfma_rate",
 )
@@ -107,6 +107,8 @@ def lib():
     L.mm_fill_weights_lane.argtypes = [c_vp, c_int, c_int, ctypes.c_uint, c_vp]
     L.mm_pack_weights.restype = c_int
     L.mm_pack_weights.argtypes = [c_vp, c_vp, c_int, c_int, c_int, c_vp]
+    L.mm_pack_weights_paired.restype = c_int
+    L.mm_pack_weights_paired.argtypes = [c_vp, c_vp, c_int, c_int, c_int, c_int, c_vp]
     L.mm_pack_weights_from_reference.restype = c_int
     L.mm_pack_weights_from_reference.argtypes = [c_vp, c_vp, c_int, c_int, c_int, c_vp]
     L.mm_fill_weights_normal.restype = c_int

@@ -41,21 +41,34 @@ fill_w_lane_kernel(uint8_t* __restrict__ w, int n_rows, int k_cols, uint32_t see
     }
 }
 
-// Logical row-major [n_mats][n_rows][k_cols] -> tile layout, 16 bytes per thread.
+// Logical row-major [n_mats][n_rows][k_cols] -> tile layout.  pair > 0: the
+// source rows are [gate; up] halves and tile row rho is row rho of the paired
+// order (gate and up alternating in blocks of `pair` rows), read in place.
+// One wave per tile: lane L reads 32 contiguous bytes of row L%16 and writes
+// the two 16-byte slots they belong to.  HBM-bound, each byte read once and
+// written once; measured on MI355X for the weights of 32 experts, H = 6144, I =
+// 2048: 2191 us with the pairing as torch copies before a 16-byte-per-thread
+// pack, 423 us with both in this kernel.
 __global__ void __launch_bounds__(256)
 pack_weights_kernel(uint8_t* __restrict__ dst, const uint8_t* __restrict__ src, int n_mats,
-                    int n_rows, int k_cols) {
+                    int n_rows, int k_cols, int pair) {
     const int KT = k_cols >> 7;
-    const size_t per_mat = (size_t)(n_rows >> 4) * KT * 128;
-    const size_t total = per_mat * n_mats;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-         i += (size_t)gridDim.x * blockDim.x) {
-        const size_t m = i / per_mat, j = i % per_mat;
-        int row, k;
-        slot_coords(j, KT, row, k);
-        const uint8_t* s = src + (m * n_rows + row) * (size_t)k_cols + k;
-        *reinterpret_cast<v4i*>(dst + i * 16) = *reinterpret_cast<const v4i*>(s);
-    }
+    const int lane = threadIdx.x & 63, kt = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (kt >= KT) return;
+    for (int m = blockIdx.z; m < n_mats; m += gridDim.z)
+        for (int nt = blockIdx.y; nt < (n_rows >> 4); nt += gridDim.y) {
+            int row = nt * 16 + (lane & 15);
+            if (pair > 0) {
+                const int blk = row / (2 * pair), r = row - blk * 2 * pair;
+                row = r < pair ? blk * pair + r : (n_rows >> 1) + blk * pair + r - pair;
+            }
+            const uint8_t* s = src + ((size_t)m * n_rows + row) * (size_t)k_cols + kt * 128 +
+                               32 * (lane >> 4);
+            const v4i lo = load16(s), hi = load16(s + 16);
+            uint8_t* d = dst + (((size_t)m * (n_rows >> 4) + nt) * KT + kt) * kTileBytes + lane * 16;
+            *reinterpret_cast<v4i*>(d) = lo;
+            *reinterpret_cast<v4i*>(d + 1024) = hi;
+        }
 }
 
 // The reference's on-device lane-tile layout -> this library's tile layout,

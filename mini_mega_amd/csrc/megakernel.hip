@@ -585,17 +585,29 @@ void fill_weights_lane(uint8_t* w, int n_rows, int k_cols, uint32_t seed, hipStr
     record(launched(kOk));
 }
 
-void pack_weights(uint8_t* dst, const uint8_t* src, int n_mats, int n_rows, int k_cols,
-                  hipStream_t s) {
+static void launch_pack(uint8_t* dst, const uint8_t* src, int n_mats, int n_rows, int k_cols,
+                        int pair, hipStream_t s) {
     if (!dst || !src) { record(kErrNullPointer); return; }
-    if (n_mats <= 0 || n_rows <= 0 || n_rows % 16 || k_cols <= 0 || k_cols % 128) {
+    if (n_mats <= 0 || n_rows <= 0 || n_rows % 16 || k_cols <= 0 || k_cols % 128 ||
+        (pair > 0 && n_rows % (2 * pair))) {
         record(kErrBadDims);
         return;
     }
-    const size_t slots = (size_t)n_mats * (n_rows / 16) * (k_cols / 128) * 128;
-    hipLaunchKernelGGL(mm::pack_weights_kernel, dim3(grid_for(slots)), dim3(256), 0, s, dst, src,
-                       n_mats, n_rows, k_cols);
+    const dim3 grid((k_cols / 128 + 3) / 4, std::min(n_rows / 16, 65535), std::min(n_mats, 65535));
+    hipLaunchKernelGGL(mm::pack_weights_kernel, grid, dim3(256), 0, s, dst, src, n_mats, n_rows,
+                       k_cols, pair);
     record(launched(kOk));
+}
+
+void pack_weights(uint8_t* dst, const uint8_t* src, int n_mats, int n_rows, int k_cols,
+                  hipStream_t s) {
+    launch_pack(dst, src, n_mats, n_rows, k_cols, 0, s);
+}
+
+void pack_weights_paired(uint8_t* dst, const uint8_t* src, int n_mats, int n_rows, int k_cols,
+                         int pair, hipStream_t s) {
+    if (pair <= 0) { record(kErrBadDims); return; }
+    launch_pack(dst, src, n_mats, n_rows, k_cols, pair, s);
 }
 
 void pack_weights_from_reference(uint8_t* dst, const uint8_t* src, int n_mats, int n_rows,
@@ -755,6 +767,12 @@ int mm_fill_weights_lane(uint8_t* w, int n_rows, int k_cols, unsigned seed, void
 int mm_pack_weights(uint8_t* dst, const uint8_t* src, int n_mats, int n_rows, int k_cols,
                     void* stream) {
     fp8mega::pack_weights(dst, src, n_mats, n_rows, k_cols, (hipStream_t)stream);
+    return fp8mega::last_error();
+}
+
+int mm_pack_weights_paired(uint8_t* dst, const uint8_t* src, int n_mats, int n_rows, int k_cols,
+                           int pair, void* stream) {
+    fp8mega::pack_weights_paired(dst, src, n_mats, n_rows, k_cols, pair, (hipStream_t)stream);
     return fp8mega::last_error();
 }
 

@@ -315,15 +315,25 @@ def _sf_to_ue8m0(sf: torch.Tensor) -> torch.Tensor:
     return ((bits >> 23) & 0xFF).to(torch.uint8)
 
 
-def pack_weights(w: torch.Tensor) -> torch.Tensor:
-    """Logical row-major fp8 [E, N, K] -> tile layout (device kernel)."""
+def pack_weights(w: torch.Tensor, pair: int = 0) -> torch.Tensor:
+    """Logical row-major fp8 [E, N, K] -> tile layout (device kernel); pair > 0:
+    [gate | up] rows are put in the paired order (blocks of `pair` rows) on the
+    way (reference _interleave_weights, mega/__init__.py:493-509)."""
     if w.dim() == 2:
         w = w.unsqueeze(0)
     e, n, k = w.shape
+    if pair and n % (2 * pair):
+        raise RuntimeError(f"{n} gate and up rows do not pair in blocks of {pair}")
     src = w.contiguous().view(torch.uint8)
+    if src.data_ptr() % 16:
+        src = src.clone()   # the kernel loads 16 bytes at a time
     dst = torch.empty_like(src)
-    check("mm_pack_weights", lib().mm_pack_weights(dst.data_ptr(), src.data_ptr(), e, n, k,
-                                                   _stream_ptr()))
+    if pair:
+        check("mm_pack_weights_paired", lib().mm_pack_weights_paired(
+            dst.data_ptr(), src.data_ptr(), e, n, k, pair, _stream_ptr()))
+    else:
+        check("mm_pack_weights", lib().mm_pack_weights(dst.data_ptr(), src.data_ptr(), e, n, k,
+                                                       _stream_ptr()))
     return dst.view(torch.float8_e4m3fn)
 
 
@@ -347,7 +357,7 @@ def transform_weights_for_mega_moe(
         s2 = None if s2 is None else s2.unsqueeze(0)
     I = w1.shape[1] // 2
     G = pairing_block(I)
-    l1_t = pack_weights(_interleave_rows(w1.view(torch.uint8), G).view(torch.float8_e4m3fn))
+    l1_t = pack_weights(w1, pair=G)
     l2_t = pack_weights(w2)
     if (s1 is None) != (s2 is None):
         raise ValueError("give scales for both l1 and l2 or for neither")

@@ -1,6 +1,7 @@
-"""GPU tests of the one-workgroup routing at the edges of its segments and
-limits, and of the activation fold beside it, against the oracle's routing and
-the fold's own kernel."""
+"""GPU tests of the small-launch paths: the one-workgroup routing at the edges
+of its segments and limits, the activation fold beside it, and weight packing
+with the gate/up pairing in the kernel.  Each against the oracle's routing or a
+plain restatement."""
 import dataclasses
 
 import numpy as np
@@ -58,3 +59,38 @@ def test_fold_beside_the_routing(T, H, scaled):
     counts, offsets, perm, pair_pos = orc.route(idx, E, None)
     assert np.array_equal(buf.counts().cpu().numpy(), counts)
     assert np.array_equal(buf.pair_pos(T).cpu().numpy().ravel(), np.asarray(pair_pos).ravel())
+
+
+# one tile column, a last workgroup of fewer than 4 column tiles, several pairs
+# of blocks, the smallest pairing block; an unaligned and a strided source
+@pytest.mark.parametrize("E,I,H", [(1, 128, 128), (3, 256, 640), (2, 768, 1152), (5, 512, 256)])
+def test_paired_packing(E, I, H):
+    G = mm.pairing_block(I)
+    rng = np.random.default_rng(I + H)
+    w1 = rng.integers(0, 127, size=(E, 2 * I, H)).astype(np.uint8)
+    w2 = rng.integers(0, 127, size=(E, H, I)).astype(np.uint8)
+    rows = inputs.paired_to_torch_rows(I)
+
+    def check(a, b):
+        p1, p2 = mm.transform_weights_for_mega_moe(a, b)
+        for e in range(E):
+            got = inputs.unpack_tiles(p1[e].view(torch.uint8).cpu().numpy().ravel(), 2 * I, H)
+            assert np.array_equal(got, w1[e][rows])
+            got = inputs.unpack_tiles(p2[e].view(torch.uint8).cpu().numpy().ravel(), H, I)
+            assert np.array_equal(got, w2[e])
+
+    a = torch.from_numpy(w1).cuda()
+    b = torch.from_numpy(w2).cuda()
+    fp8 = torch.float8_e4m3fn
+    check(a.view(fp8), b.view(fp8))
+    off = torch.empty(a.numel() + 3, dtype=torch.uint8, device="cuda")[3:].view(a.shape)
+    off.copy_(a)
+    check(off.view(fp8), b.view(fp8))
+    check(a.transpose(1, 2).contiguous().transpose(1, 2).view(fp8), b.view(fp8))
+
+
+def test_rows_that_do_not_pair_are_refused():
+    w1 = torch.zeros((1, 2 * 384, 128), dtype=torch.uint8, device="cuda")   # 384 % 256 != 0
+    w2 = torch.zeros((1, 128, 384), dtype=torch.uint8, device="cuda")
+    with pytest.raises(RuntimeError):
+        mm.transform_weights_for_mega_moe(w1.view(torch.float8_e4m3fn), w2.view(torch.float8_e4m3fn))
