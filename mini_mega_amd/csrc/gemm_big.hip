@@ -25,7 +25,7 @@
 //     register pipeline and converts them exactly to bf16;
 //   * v_mfma_f32_16x16x32_bf16 (fp32-accurate sums; see gemm.hip) over the
 //     item's NT active token tiles -- NT is a compile-time specialisation
-//     picked per item (1..16), so the k loop has no branch
+//     picked per item (1..17), so the k loop has no branch
 //     and the accumulator chains are independent;
 //   * epilogues as in gemm.hip: L1 SwiGLU + fp8 (raw, or per-128 UE8M0 with
 //     the 128-column amax reduced over the waves in LDS), L2 bf16.
@@ -53,7 +53,8 @@ constexpr int kXOddPad = 16;   // LDS shift of the odd 16-byte columns (x_swizzl
 constexpr int kXTileBytes = 16 * kTileK * 2 + kXOddPad;   // one bf16 token tile: 16 rows x 128 k
 constexpr int kXTile8Bytes = kTileBytes + kXOddPad;       // the same in fp8
 constexpr int kBlockTiles = 16;                 // weight tiles = 256 rows per workgroup
-constexpr int kBigRows = kBigMaxTiles * 16;     // token rows per work item (max)
+constexpr int kBodyTiles = kBigMaxTiles + 1;    // token tiles of a unit (max; see unit_rows)
+constexpr int kBigRows = kBodyTiles * 16;       // token rows of a unit (max)
 static_assert(kBlockTiles * 16 == kL2BlockN && kBlockTiles * 8 == kL1BlockH, "block shape");
 
 // Workgroup shape: W waves, kWT = 16 / W weight tiles per wave.
@@ -70,7 +71,7 @@ struct Geo {
 constexpr int kSfxPitch = kBigMaxKT + 16;
 
 struct alignas(16) BigSmem {
-    uint8_t x[2][kBigMaxTiles * kXTileBytes];   // bf16 tiles, double buffered
+    uint8_t x[2][kBodyTiles * kXTileBytes];   // bf16 tiles, double buffered
     uint8_t sfx[kBigRows][kSfxPitch];           // the item's row scales [row][k-step]
     uint32_t tok[kBigRows];                      // L1: the token of each item row
     uint8_t sfw[kBigMaxKT][kBlockTiles];        // the block's weight-tile scales [k-step][tile]
@@ -755,6 +756,25 @@ __device__ __forceinline__ bool big_unit(const GemmParams& p, int nb, BigItem& i
     it.e = v.x;
     it.m0 = v.y;
     it.rows = v.z - v.y;
+    // An expert whose rows fit fewer units of kBigRows than it has items of 256
+    // (257 to 272 rows, 513 to 544, ..) runs as that many units of equal
+    // rows, and the last of its units end here: 17 token tiles in one unit cost
+    // less than 9 + 8 in two, which stream the weights twice.  (The empty units
+    // come last, not in turn with the others: workgroups go round the shader
+    // engines, and every second one empty left half of them idle.)  Measured on
+    // MI355X: 272 rows on every expert, L1 / L2 2990 / 1635 -> 2691 / 1429 us (fp8 MFMA
+    // 2052 / 1121 -> 1776 / 991); T = 8192 (a third of the experts) layer 4320 -> 4147.
+    if (p.merge && n != 1) {
+        const int m0 = items[i0].y, rows = items[i0 + n - 1].z - m0;
+        const int n2 = (rows + kBigRows - 1) / kBigRows;
+        if (n2 < n) {
+            if (local >= nb * n2) return false;
+            const int sz = (rows + n2 - 1) / n2, j = local % n2;
+            it.bx = local / n2;
+            it.m0 = m0 + j * sz;
+            it.rows = min(sz, rows - j * sz);
+        }
+    }
     return true;
 }
 
@@ -798,7 +818,7 @@ __device__ __forceinline__ void big_load_scales(BigSmem& sm, int KT, int nrows, 
     __syncthreads();
 }
 
-// NT as run for an item of `tiles` (<= kBigMaxTiles) token tiles: exact, so
+// NT as run for an item of `tiles` (<= kBodyTiles) token tiles: exact, so
 // that the MFMAs cover no more than the item's partial last tile (at T =
 // 8192 rounding to even counts above 8 tiles ran 6% more MFMA work: padding
 // 11.7% vs 5.2% of the routed rows; layer 5122 -> 4782 us on MI355X).
@@ -819,7 +839,8 @@ __device__ __forceinline__ void big_load_scales(BigSmem& sm, int KT, int nrows, 
         case 13: BODY(13); break; \
         case 14: BODY(14); break; \
         case 15: BODY(15); break; \
-        default: BODY(16); break; \
+        case 16: BODY(16); break; \
+        default: BODY(17); break; \
     }
 
 // ---------------------------------------------------------------------- L1 --

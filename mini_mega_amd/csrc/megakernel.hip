@@ -266,6 +266,7 @@ int do_l1(const MegaLaunchArgs& a, Stage stage, hipStream_t s) {
     p.xcd_cuts = p.status + mm::kCutsL1;
     p.queue = at<int>(b, b.L.status) + mm::kQueueL1;
     p.other_queue = at<int>(b, b.L.status) + mm::kQueueL2;
+    p.merge = b.m_tile == 16 * mm::kBigMaxTiles;
     p.self_reset = stage == Stage::kAlone;
     p.tail_ord = reinterpret_cast<const uint8_t*>(p.status + mm::kTailOrdL1);
     const int nb = a.intermediate / mm::kL1BlockH;
@@ -289,6 +290,7 @@ int do_l2(const MegaLaunchArgs& a, Stage stage, hipStream_t s) {
     p.queue = at<int>(b, b.L.status) + mm::kQueueL2;
     const int nb = a.hidden / mm::kL2BlockN;
     p.other_queue = at<int>(b, b.L.status) + mm::kQueueL1;
+    p.merge = b.m_tile == 16 * mm::kBigMaxTiles;
     p.self_reset = stage == Stage::kAlone;
     int grid = big_grid(a, b, nb, stage == Stage::kRouted);
     // The walk is offered for 17 to 128 routed rows per expert on average;

@@ -94,6 +94,7 @@ struct GemmParams {
     int ready_target;         // L1 blocks per item (L2 waits for this count)
     int spin_limit;           // L2: polls of a ready counter before giving up
     int* err;                 // status word [0]: kStatusWaitTimeout on give-up
+    int merge;                // 1: the items are full windows (256 rows), see big_unit
     // L2: workgroups of the walk (0: never); the device runs the units as the
     // walk or one per workgroup (walk_taken decides from the item size)
     int walk;

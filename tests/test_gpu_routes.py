@@ -1,7 +1,7 @@
-"""GPU tests of the small-launch paths: the one-workgroup routing at the edges
-of its segments and limits, the activation fold beside it, and weight packing
-with the gate/up pairing in the kernel.  Each against the oracle's routing or a
-plain restatement."""
+"""GPU tests of dispatch edges: the one-workgroup routing at the edges of its
+segments and limits, the activation fold beside it, weight packing with the
+gate/up pairing in the kernel, and units of up to 17 token tiles.  Each against
+the oracle, a plain restatement or the general path."""
 import dataclasses
 
 import numpy as np
@@ -94,3 +94,38 @@ def test_rows_that_do_not_pair_are_refused():
     w2 = torch.zeros((1, 128, 384), dtype=torch.uint8, device="cuda")
     with pytest.raises(RuntimeError):
         mm.transform_weights_for_mega_moe(w1.view(torch.float8_e4m3fn), w2.view(torch.float8_e4m3fn))
+
+
+# rows around the largest one-unit size (272) and its multiples, and around the
+# 256-row items: 257-272 run as one unit, 513-544 as two, the others as items
+@pytest.mark.parametrize("rows", [[256, 257, 264, 272, 273], [512, 513, 544, 545, 1, 0, 271]])
+@pytest.mark.parametrize("scaled", [True, False])
+def test_units_of_seventeen_token_tiles(rows, scaled):
+    """Against the oracle at the staged tolerances, and bit for bit against the
+    one-launch form, which runs the items as they are; the fp8 MFMA path
+    against its own result on 64-row windows (same sums, other units)."""
+    E, K, H, I = len(rows), 1, 512, 256
+    ids = np.repeat(np.arange(E), rows)
+    np.random.default_rng(5).shuffle(ids)
+    T = ids.size
+    idx = ids.reshape(T, 1).astype(np.int64)
+    wts = np.full((T, 1), 0.75, np.float32)
+    c = mc.normal_case(E, K, H, I, T, seed=17, scaled=scaled, idx=idx, wts=wts)
+    r = mc.run_layer(c)
+    mc.check_routing(c, r)
+    for e in range(E):
+        if rows[e]:
+            mc.check_l1(c, r, e, max_rows=None)
+            mc.check_l2(c, r, e, max_rows=None)
+    mc.check_reduce(c, r)
+    r.buf.fuse_l1l2 = True
+    one = mc.run_layer(c, buf=r.buf)
+    assert np.array_equal(one.y32.view(np.uint32), r.y32.view(np.uint32))
+    r.buf.fuse_l1l2 = False
+    r.buf.mfma_fp8 = True
+    f8 = mc.run_layer(c, buf=r.buf)
+    buf = mm.get_symm_buffer_for_mega_moe(None, E, T, K, H, I, expert_window=64)
+    buf.write_fp32_y = True
+    buf.mfma_fp8 = True
+    f8w = mc.run_layer(dataclasses.replace(c, win=64), buf=buf)
+    assert np.array_equal(f8.y32.view(np.uint32), f8w.y32.view(np.uint32))
