@@ -251,6 +251,16 @@ const GemmKernel kL2Small[2] = {mm::l2_kernel<1>, mm::l2_kernel<2>};
 // previous one's routing.
 enum class Stage { kAlone, kReused, kRouted };
 
+// A GEMM that is launched alone starts from a zeroed tail queue whatever ran
+// before it: L2's is spent after a launch_compute that no combine followed, and
+// tickets from a spent queue would leave the last units of every range undone.
+// Inside launch_compute the launches around a GEMM zero its queue, at no launch
+// of their own.
+void zero_queue(Stage stage, int m_tile, int* queue, hipStream_t s) {
+    if (stage == Stage::kAlone && m_tile > 32)
+        hipLaunchKernelGGL(mm::fill_int_kernel, dim3(1), dim3(256), 0, s, queue, mm::kQueueInts, 0);
+}
+
 int do_l1(const MegaLaunchArgs& a, Stage stage, hipStream_t s) {
     Bound b;
     int st = bind(a, b, true);
@@ -270,6 +280,7 @@ int do_l1(const MegaLaunchArgs& a, Stage stage, hipStream_t s) {
     p.self_reset = stage == Stage::kAlone;
     p.tail_ord = reinterpret_cast<const uint8_t*>(p.status + mm::kTailOrdL1);
     const int nb = a.intermediate / mm::kL1BlockH;
+    zero_queue(stage, b.m_tile, p.queue, s);
     launch_gemm(kL1Small, a.mfma_fp8 ? mm::l1_big_f8_kernel : mm::l1_big_kernel, b.m_tile, nb,
                 b.L.max_items, big_grid(a, b, nb, stage == Stage::kRouted), s, p);
     return launched(kOk);
@@ -305,6 +316,7 @@ int do_l2(const MegaLaunchArgs& a, Stage stage, hipStream_t s) {
         p.walk = cu_count() < 8 ? 8 : cu_count();
         if (grid < p.walk) grid = p.walk;
     }
+    zero_queue(stage, b.m_tile, p.queue, s);
     launch_gemm(kL2Small, a.mfma_fp8 ? mm::l2_big_f8_kernel : mm::l2_big_kernel, b.m_tile, nb,
                 b.L.max_items, grid, s, p);
     return launched(kOk);

@@ -51,11 +51,13 @@ constexpr int kCutsL2 = 32;         // status[32..40]: the same for L2
 // Tail queues of the big GEMMs: per XCD a ticket counter over the last
 // kQueueTail units of its range (ranges of more than 2 * kQueueTail units),
 // plus a count of the workgroups that took tickets (status[44..52] for L1,
-// [53..61] for L2; zeroed by the routing scan and again after each GEMM, see
-// gemm_big.hip).  L1 always takes
-// tickets, L2 when its largest item has more than 32 rows (gemm_big.hip:
-// big_unit<true>).  L1's tickets go out costliest unit first: the routing
-// scan writes each tail's order (kTailOrdL1); L2's go out in unit order.
+// [53..61] for L2).  Who zeroes them: the routing, both; every L2 launch, L1's;
+// every L1 launch and the combine, L2's; a GEMM launched alone, its own, before
+// it starts and by its last ticket taker.  So L1's are zero between the entry
+// points, and L2's are spent after a launch_compute until the next launch.  L1
+// always takes tickets, L2 when its largest item has more than 32 rows
+// (gemm_big.hip: big_unit<true>).  L1's tickets go out costliest unit first: the
+// routing scan writes each tail's order (kTailOrdL1); L2's go out in unit order.
 constexpr int kQueueInts = 9;
 constexpr int kQueueL1 = 44;
 constexpr int kQueueL2 = kQueueL1 + kQueueInts;

@@ -1,7 +1,9 @@
 """GPU tests of dispatch edges: the one-workgroup routing at the edges of its
 segments and limits, the activation fold beside it, weight packing with the
-gate/up pairing in the kernel, and units of up to 17 token tiles.  Each against
-the oracle, a plain restatement or the general path."""
+gate/up pairing in the kernel, units of up to 17 token tiles, and the GEMMs
+launched alone after whatever ran before.  Each against the oracle, a plain
+restatement or the general path."""
+import ctypes
 import dataclasses
 
 import numpy as np
@@ -129,3 +131,69 @@ def test_units_of_seventeen_token_tiles(rows, scaled):
     buf.mfma_fp8 = True
     f8w = mc.run_layer(dataclasses.replace(c, win=64), buf=buf)
     assert np.array_equal(f8.y32.view(np.uint32), f8w.y32.view(np.uint32))
+
+
+@pytest.mark.parametrize("mfma_fp8", [False, True])
+def test_gemms_launched_alone_after_anything(mfma_fp8):
+    """launch_l1 / launch_l2 run every unit whatever ran before: after a
+    launch_compute that no combine followed (its L2 leaves the tail queue
+    spent), and after themselves.  About 300 rows per expert, so that both
+    GEMMs take tickets in every XCD range."""
+    E, K, H, I, T = 32, 8, 6144, 2048, 1200
+    c = mc.normal_case(E, K, H, I, T, seed=71)
+    other_w2 = inputs.make_weights_normal(E, H, I, seed=72)[1]
+    r = mc.run_layer(c)
+    buf, L, s = r.buf, mm.lib(), torch.cuda.current_stream().cuda_stream
+    buf.mfma_fp8 = mfma_fp8
+    nitems, max_rows = int(r.status[1]), int(r.status[5])
+    # a range of more than 64 units has a tail; the walk, which has none, is out
+    assert max_rows > 128 and nitems * min(I // 128, H // 256) // 8 > 64
+    y = torch.empty((T, H), dtype=torch.bfloat16, device="cuda")
+
+    def args(l2=(c.w2, c.s2), **kw):
+        a = buf.make_args(T, (c.w1, c.s1), l2, y_bf16=y)
+        for k, v in kw.items():
+            setattr(a, k, v)
+        return ctypes.byref(a)
+
+    def ffn():
+        return buf.ffn(T * K).clone(), buf.ffn_sf(T * K).clone()
+
+    def clear(off):
+        buf.workspace[int(off):].zero_()
+
+    def queues_zero():
+        return not bool(buf.status()[44:62].any())
+
+    assert L.mm_launch_full(args(other_w2), s) == 0
+    want_other = buf.l2_out(T * K).clone()
+    assert L.mm_launch_full(args(), s) == 0
+    want_ffn, want_l2 = ffn(), buf.l2_out(T * K).clone()
+    assert not torch.equal(want_l2, want_other)
+
+    for before in (lambda: L.mm_launch_compute(args(), s),
+                   lambda: L.mm_launch_full(args(skip_combine=1), s),
+                   lambda: L.mm_launch_compute(args(skip_prologue=1), s)):
+        assert before() == 0
+        clear(buf.layout.l2)
+        assert L.mm_launch_l2(args(), s) == 0
+        assert torch.equal(buf.l2_out(T * K), want_l2)
+        assert before() == 0
+        assert L.mm_launch_l2(args(other_w2), s) == 0
+        assert torch.equal(buf.l2_out(T * K), want_other)
+        assert queues_zero()
+    assert L.mm_launch_compute(args(), s) == 0
+    for _ in range(2):
+        clear(buf.layout.ffn)
+        assert L.mm_launch_l1(args(), s) == 0
+        assert all(torch.equal(a, b) for a, b in zip(ffn(), want_ffn))
+        assert queues_zero()
+    for _ in range(2):
+        clear(buf.layout.l2)
+        assert L.mm_launch_l2(args(), s) == 0
+        assert torch.equal(buf.l2_out(T * K), want_l2)
+        assert queues_zero()
+    # and a compute on that routing after them
+    clear(buf.layout.ffn)
+    assert L.mm_launch_compute(args(skip_prologue=1), s) == 0
+    assert torch.equal(buf.l2_out(T * K), want_l2)
