@@ -53,7 +53,7 @@ constexpr int kXOddPad = 16;   // LDS shift of the odd 16-byte columns (x_swizzl
 constexpr int kXTileBytes = 16 * kTileK * 2 + kXOddPad;   // one bf16 token tile: 16 rows x 128 k
 constexpr int kXTile8Bytes = kTileBytes + kXOddPad;       // the same in fp8
 constexpr int kBlockTiles = 16;                 // weight tiles = 256 rows per workgroup
-constexpr int kBodyTiles = kBigMaxTiles + 1;    // token tiles of a unit (max; see unit_rows)
+constexpr int kBodyTiles = kBigMaxTiles + 1;    // token tiles of a unit (max; see big_unit)
 constexpr int kBigRows = kBodyTiles * 16;       // token rows of a unit (max)
 static_assert(kBlockTiles * 16 == kL2BlockN && kBlockTiles * 8 == kL1BlockH, "block shape");
 
@@ -921,7 +921,8 @@ __device__ __forceinline__ void l1_big_body(const GemmParams& p, const BigItem& 
     const int I128 = I >> 7;
     if (p.ffn_ue8m0) {
         // amax over the block's 128 hidden columns = the W waves; the LDS
-        // tiles are free after the main loop's last barrier.
+        // tiles are free after the main loop's last barrier (what slower waves
+        // still read there is never used, see l2_store_tile).
         float* red = reinterpret_cast<float*>(&sm.x[0][0]);   // [W][kBigRows]
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
@@ -1030,8 +1031,13 @@ __global__ void __launch_bounds__(512) l1_big_f8_kernel(GemmParams p) {
 // L2 epilogue: the unit's bf16 tile (rows x 256 channels) goes through LDS so
 // that every global store writes whole rows (a wave: two 512-byte rows per
 // instruction) instead of 32-byte pieces of 16 rows from the MFMA layout.
-// The caller's main loop ended on a barrier; the tile (<= 256 rows at a
-// 528-byte pitch, 132 KiB) overlays the LDS operand tiles and the scales.
+// The tile (up to 272 rows at a 528-byte pitch, 140 KiB) overlays the LDS
+// operand tiles and the scales, with no barrier before its first write: after
+// the main loop's last barrier (bf16: kReadAhead chunks before the loop's end)
+// a wave that is still in the loop reads from LDS only the operands ahead of
+// the last k-step, which nothing uses, and writes nothing there.  A k-step that
+// used anything read after that barrier, or read a scale there, would need a
+// barrier here and before L1's amax scratch.
 // The pitch is 132 dwords, 4 banks past a multiple of 64: the 16 rows of a
 // quarter-wave's 8-byte writes fall in distinct banks (measured on MI355X at
 // T = 8192 / 2048: L2's LDS bank conflicts halved against a 544-byte pitch,
