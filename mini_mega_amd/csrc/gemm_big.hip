@@ -667,9 +667,10 @@ struct BigItem {
 // tiles), and saved 2-4% of L2 at T = 8192 (1571-1586 vs 1603-1612 us) and
 // with Zipf(1.1) skew at T = 2048 (651-663 vs 678-679 us), so L2 takes
 // tickets only when its largest item has more than 32 rows (at T = 2048 the
-// walk runs those launches).  L1's tickets go out costliest unit first (by
-// the token tiles of the unit's item; the order is the routing scan's
-// tail_ord), so that no heavy unit starts after the light ones of its tail:
+// walk runs those launches).  L1's tickets go out by the token tiles of the
+// unit's item, most first (the routing scan's tail_ord), so that a heavy item's
+// unit does not start after the light ones of its tail (a unit of 17 tiles
+// ranks as its items of 9, even in time, see route.hip):
 // Zipf(1.1) T = 2048 L1 1193-1195 vs 1223-1231 us, T = 512 / 2048 / 8192
 // even (measured on MI355X).  L2's tickets gained nothing from the order
 // and go out in unit order.

@@ -56,15 +56,16 @@ constexpr int kCutsL2 = 32;         // status[32..40]: the same for L2
 // it starts and by its last ticket taker.  So L1's are zero between the entry
 // points, and L2's are spent after a launch_compute until the next launch.  L1
 // always takes tickets, L2 when its largest item has more than 32 rows
-// (gemm_big.hip: big_unit<true>).  L1's tickets go out costliest unit first: the
-// routing scan writes each tail's order (kTailOrdL1); L2's go out in unit order.
+// (gemm_big.hip: big_unit<true>).  L1's tickets go out by the token tiles of the
+// units' items, most first: the routing scan writes each tail's order
+// (kTailOrdL1); L2's go out in unit order.
 constexpr int kQueueInts = 9;
 constexpr int kQueueL1 = 44;
 constexpr int kQueueL2 = kQueueL1 + kQueueInts;
 constexpr int kQueueTail = 32;      // units per XCD handed out by ticket (one per CU)
 constexpr int kStealers = 8;        // workgroups per XCD past its range that take others' tickets
 static_assert(kQueueTail * 8 <= (kStatusInts - kTailOrdL1) * 4, "the tail order fits");
-constexpr int kTailOrderRows = 128;   // L1's tail order is costliest-first above this item size
+constexpr int kTailOrderRows = 128;   // L1's tail order is by token tiles above this item size
 
 // Parameters of the two grouped GEMMs (one struct so that the launcher and
 // the kernels agree on one argument list).

@@ -131,7 +131,16 @@ __device__ void route_finish(RouteSmem& sh, int run, int P, int E, int cap, int 
     // and a weight block's k-step streams in ~1.23 us).  XCD x starts where
     // the running cost crosses x/8 of the total (the same expert for L1 and
     // L2, whose costs differ by the factor nb); each range is then clamped to
-    // its share of the grid, nb * max_items + 8 workgroups.
+    // its share of the grid, nb * max_items + 8 workgroups.  (The constants were
+    // fitted before big_step spread its loads, on the bf16 path; the fp8 path
+    // uses them too.)
+    // An expert whose items big_unit runs as fewer units of up to 17 token tiles
+    // is planned as its items here and in the tail order below: two units of
+    // 9 tiles, say, for one of 17 and an empty one.  Planned as they run (measured on
+    // MI355X, as it is vs the order alone vs the cuts as well, all even): T =
+    // 8192 4168 vs 4173 vs 4167 us, Zipf(1.1) 4387 vs 4394 vs 4384, Zipf(1.1) T =
+    // 2048 1834 vs 1837 vs 1831; fp8 path T = 8192 2876 vs 2871 vs 2880, Zipf(1.1)
+    // 3098 vs 3096 vs 3086.
     const int uc = max(9, 2 + min((sz + 15) >> 4, kBigMaxTiles));
     const int w = nm * uc;
     __syncthreads();   // sh.rows
@@ -211,9 +220,11 @@ __device__ void route_finish(RouteSmem& sh, int run, int P, int E, int cap, int 
         }
     }
     // Ticket order of L1's tail queues (the last t = min(range, kQueueTail)
-    // units of each XCD range): costliest unit first, i.e. by the token tiles
-    // of its item, descending, ties in unit order, so that heavy units do not
-    // start after light ones at the end of the kernel.  Tail unit i of XCD x
+    // units of each XCD range; only a range of more than 2 * kQueueTail units
+    // reads it): by the token tiles of the unit's item, descending, ties in unit
+    // order, so that the units of heavy items do not start after light ones at
+    // the end of the kernel (units of 17 tiles rank as their items, above).
+    // Tail unit i of XCD x
     // is unit cuts[x + 1] - t + i; L1 runs ticket k as tail unit order[k]
     // (gemm_big.hip: claim_tail_unit).  One thread per tail slot finds its
     // unit's expert by binary search over the item offsets.  Only when some
