@@ -533,8 +533,12 @@ __device__ __forceinline__ void w_load8(WStage8<WT>& w, const WTiles<WT>& wt, in
 // One k-step: NT chunks, chunk j = token tile j: the LDS read of the operand
 // D tiles ahead (two 16-byte halves and its row scale), a share of the
 // commit of k-step kt+1 (spread over all chunks: the rows were loaded a step
-// earlier; measured even with the second half or last quarter, and the only
-// placement without spills in L1), and kWT MFMAs.
+// earlier; measured even with the second half or last quarter), and kWT MFMAs.
+// L1's 17-tile body keeps 3 values in scratch memory across its loop, stored
+// before it and reloaded after it.  Bodies without them were slower (measured on
+// MI355X, 272 rows on every expert, layer 2926 us): one operand ahead 2997, one
+// activation stage 2942; the fifth chunk alone with one stage and the thread
+// index read anew in the epilogue 2988 against 2959 on another box.
 template <int W, int NT, int S, int s, class XL>
 __device__ __forceinline__ void big_step_f8(v4f (&acc)[Geo<W>::kWT][NT], BigSmem& sm, XL& xl,
                                             WStage8<Geo<W>::kWT> (&w)[S],
