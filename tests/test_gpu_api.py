@@ -329,10 +329,10 @@ def test_l2_walk_matches_one_unit_kernel(E, K, H, I, T, zipf, win, scaled, walks
     """The L2 walk (one workgroup per CU, the next unit's weights streamed during
     the current one) runs when the largest work item has 3..8 token tiles and
     I / 128 is a multiple of 4 (the host tries it above 16 routed rows per
-    expert on average); otherwise the one-unit-per-workgroup kernel launched
-    after it does.  y, the ffn bytes and the L2 rows are bit-identical with the
-    walk disabled (l2_no_walk), including split experts (a 128-row window under
-    skew) and the raw path; a graph of two launches replays to the same y."""
+    expert on average); otherwise the kernel runs one unit per workgroup.  y, the
+    ffn bytes and the L2 rows are bit-identical with the walk disabled
+    (l2_no_walk), including split experts (a 128-row window under skew) and the
+    raw path; a graph of two launches replays to the same y."""
     _say(f"L2 walk E={E} T={T} zipf={zipf} win={win} scaled={scaled}")
     c = mc.normal_case(E, K, H, I, T, seed=T + 11, scaled=scaled, zipf=zipf, win=win)
     buf = mm.get_symm_buffer_for_mega_moe(None, E, T, K, H, I, expert_window=win)
@@ -358,7 +358,7 @@ def test_l2_walk_matches_one_unit_kernel(E, K, H, I, T, zipf, win, scaled, walks
         for g, w, name in zip(got, want, ("y", "ffn", "l2")):
             assert np.array_equal(g, w), f"walk launch {rep}: {name} differs"
     assert buf.device_status()["error"] == 0
-    # two launches (walk and one-unit kernel each) as one graph, replayed twice
+    # two launches as one graph, replayed twice
     ys = [torch.empty((T, H), dtype=torch.bfloat16, device="cuda") for _ in range(2)]
     s = torch.cuda.Stream()
     s.wait_stream(torch.cuda.current_stream())

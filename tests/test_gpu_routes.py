@@ -197,3 +197,45 @@ def test_gemms_launched_alone_after_anything(mfma_fp8):
     clear(buf.layout.ffn)
     assert L.mm_launch_compute(args(skip_prologue=1), s) == 0
     assert torch.equal(buf.l2_out(T * K), want_l2)
+
+
+@pytest.mark.parametrize("mfma_fp8", [False, True])
+@pytest.mark.parametrize("T", [40, 200])
+def test_few_tokens_in_a_large_workspace(T, mfma_fp8):
+    """A launch sized by its tokens, in a workspace for many more, with tickets
+    and stealers in both GEMMs (about 64 active experts: over 64 units of L1 and
+    of L2 on each XCD; T rows on one expert): bit for bit the same tokens in a
+    workspace made for them, whose grid is the general one."""
+    E, K, H, I = 64, 8, 2560, 2048
+    rng = np.random.default_rng(T)
+    idx = np.stack([rng.permutation(E - 1)[:K] for _ in range(T)]).astype(np.int64)
+    idx[:8, :] = np.arange(64).reshape(8, 8) % (E - 1)   # nearly all are active
+    idx[:, 0] = E - 1                                    # and one holds T rows
+    c = mc.normal_case(E, K, H, I, T, seed=T + 3, idx=idx,
+                       wts=np.full((T, K), 1.0 / K, np.float32))
+    runs = []
+    for cap in (T, 8192):
+        buf = mm.get_symm_buffer_for_mega_moe(None, E, cap, K, H, I)
+        buf.mfma_fp8 = mfma_fp8
+        r = mc.run_layer(c, buf=buf)
+        assert int(r.status[5]) == T > 32
+        for base in (16, 32):
+            assert int(np.diff(r.status[base:base + 9]).min()) > 64
+        n = T * K
+        runs.append((r.y32.view(np.uint32), buf.ffn(n).cpu().numpy(), buf.ffn_sf(n).cpu().numpy(),
+                     buf.l2_out(n).cpu().numpy()))
+    assert all(np.array_equal(a, b) for a, b in zip(*runs))
+
+
+# L1 ranges of exactly 64 units (no tail queue) and of 66 (the last 32 by ticket)
+@pytest.mark.parametrize("active", [32, 33])
+def test_ranges_around_the_smallest_with_a_tail(active):
+    E, K, H, I, T = 40, 1, 256, 2048, 200
+    idx = (np.arange(T) % active).astype(np.int64).reshape(T, 1)
+    c = mc.normal_case(E, K, H, I, T, seed=active, idx=idx, wts=np.full((T, 1), 0.5, np.float32))
+    r = mc.run_layer(c)
+    assert int(np.diff(r.status[16:25]).max()) == 2 * active
+    mc.check_routing(c, r)
+    for e in range(active):
+        mc.check_l1(c, r, e, max_rows=None)
+    mc.check_reduce(c, r)
