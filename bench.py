@@ -282,7 +282,11 @@ def graph_min5(torch, mm, L, a, n=10):
 def run_config(torch, mm, inputs, L, stream, w, T, zipf, seed, steps, warmup, kernel_iters,
                fuse=False, mfma_fp8=False):
     """One workload: fresh inputs and buffer, warmup, `steps` timed layers,
-    then each stage timed alone (the routing stays valid in the workspace)."""
+    then each stage timed alone (the routing stays valid in the workspace).
+    The GEMMs' entry points zero their tail queue in a launch of their own and
+    count its takers, which launch_full does not: their figures hold about 5 us
+    more than the kernel, whose own time is within 2% of that in the layer
+    (kernel traces in profiles/)."""
     (w1, s1), (w2, s2) = w
     _, xq, xsf = inputs.make_x(T, H, seed=seed, scaled=True)
     idx, wts = inputs.route(T, E, K, seed=seed + 2, zipf_s=zipf)

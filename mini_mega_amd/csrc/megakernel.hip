@@ -3,9 +3,10 @@
 // extern "C" layer.  Reference counterpart: src/megakernel.cu:1-284 (launch
 // entry points) and test/mega_common.cuh:69-88,344-376 (geometry / args).
 //
-// Nothing here allocates or reads the environment, and only read_status
-// synchronises: every launch entry point only validates its arguments and
-// enqueues kernels on `stream`, so the layer is capture-safe.  The workspace
+// Nothing here allocates, and only read_status synchronises: every launch entry
+// point only validates its arguments, reads the reference's two environment
+// switches (env_on) and enqueues kernels on `stream`, so the layer is
+// capture-safe.  The workspace
 // is caller-owned, or (mm_launch_full_noalloc) the file-scope `scratch`.
 #include <algorithm>
 #include <cstddef>
