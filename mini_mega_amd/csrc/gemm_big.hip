@@ -300,9 +300,9 @@ struct StepCarry {
 // buffer: every wave's reads are done by then) stands before chunk kBar, D
 // chunks before the end, so that the next step's first operand reads run
 // under the last chunks' MFMAs.
-// What bounds it: at 16 token tiles the matrix cores are busy 67% of the
-// cycles, and power holds the clock at 1.9 GHz (MFMAs alone, on the same kind
-// of data, run at 2.15 GHz).  So instructions and LDS accesses saved count
+// What bounds it: at T = 8192 the matrix cores are busy 63% of L1's cycles, and
+// power holds the clock at 1.86 GHz (MFMAs alone run at 2.06-2.10 GHz, the
+// memory-bound T = 512 GEMMs at 2.3).  So instructions and LDS accesses saved count
 // even where they overlap, and deeper prefetch does not: 7 operand reads
 // ahead, 3 weight stages or 2 activation stages above 12 tiles were all even.
 // Measured on MI355X (L1 / L2 us, 256 experts, H = 6144, I = 2048, equal rows
